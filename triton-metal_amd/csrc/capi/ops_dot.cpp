@@ -201,8 +201,8 @@ int dot_impl(const char* op, const void* A, const void* B, void* C, const void* 
                        (int)st[7], bt, out_dtype, stream);
   }
   // 16-bit, no epilogue, one batch, k- and n-contiguous rows, output in the
-  // input dtype or fp32: the dense selection's MFMA tile kernels, when it has
-  // one for these sizes and alignments
+  // input dtype or fp32: the dense selection, when it has an MFMA tile kernel
+  // for these sizes and alignments
   if (is_half(in_dtype) && (out_dtype == in_dtype || out_dtype == TM_DT_F32) &&
       epilogue == TM_EPI_NONE && batch == 1 && K > 0 && st[2] == 1 && st[8] == 1 &&
       (st[5] == 1 || st[4] == 1) && fits(st[1]) && fits(st[4]) && fits(st[5]) && fits(st[7])) {
@@ -214,6 +214,16 @@ int dot_impl(const char* op, const void* A, const void* B, void* C, const void* 
                                 out_dtype, stream, &used);
       if (used || rc) return rc;
     }
+  }
+  // 16-bit and e4m3 / e5m2 operands in aligned 16-byte pieces along k or along
+  // the rows, any batch and add epilogue: the pipelined kernels
+  if (!rows_kernel && (epilogue == TM_EPI_NONE || add)) {
+    MmCall c = {A, B, add ? Z : nullptr, C, batch, M, N, K,
+                st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7], st[8],
+                st[9], epilogue == TM_EPI_ADD_COLS ? 0 : st[10],
+                epilogue == TM_EPI_ADD_ROWS ? 0 : st[11], in_dtype, out_dtype, z_dtype};
+    MmPlan pl;
+    if (mm_plan(c, &pl)) return mm_launch(c, pl, stream);
   }
   if (rows_kernel) {
     static Kernel kr("dot_rows");

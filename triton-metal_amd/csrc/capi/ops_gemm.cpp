@@ -350,11 +350,20 @@ struct GemmPlan {
   char name[96];
   unsigned grid, block;
   bool general;  // not a dense tile kernel: tm_dot, or gemm_general (K = 0)
+  bool pipe;     // a pipelined kernel, with this plan
+  MmPlan mm;
 };
+
+// The dense call as one of the pipelined products (B [K, N], or [N, K] with bt).
+MmCall mm_call(const void* A, const void* B, void* C, const void* bias, int M, int N, int K,
+               int lda, int ldb, int ldc, bool bt, int idt, int odt) {
+  return MmCall{A, B, bias, C, 1, M, N, K, 0, lda, 1, 0, bt ? 1 : ldb, bt ? ldb : 1, 0, ldc, 1,
+                0, 0, 1, idt, odt, idt};
+}
 
 void gemm_plan(int M, int N, int K, int lda, int ldb, int ldc, bool bt, bool bias, int idt,
                int odt, bool ab16, bool c16, GemmPlan* pl) {
-  pl->general = false;
+  pl->general = pl->pipe = false;
   if (idt == TM_DT_F32) {
     // fp32 inputs (the reference's default dtype): 64 x 64 tiles on the fp32
     // MFMA (gemm_f32.hip); 16-byte operand pieces when A and B are 16-byte
@@ -374,13 +383,40 @@ void gemm_plan(int M, int N, int K, int lda, int ldb, int ldc, bool bt, bool bia
   const bool mfma = is_half(idt) && (odt == idt || odt == TM_DT_F32) && K % 8 == 0 &&
                     lda % 8 == 0 && ldb % 8 == 0 && ab16 && (bt || N % 8 == 0);
   if (mfma) {
+    const long t32s = (M % 32 == 0 && N % 32 == 0) ? (long)(M / 32) * (N / 32) : 0;
+    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+    const long t256 = (M % 256 == 0 && N % 256 == 0) ? (long)(M / 256) * (N / 256) : 0;
+    // The pipelined kernels (gemm_pipe.h), except where there is too little to
+    // pipeline (us here / there, bf16, one box): one k step (K <= 64: 1024 x 832
+    // 3.4 / 3.3, 4096 x 4096 12.1 / 12.8); two of them with weights [N, K]
+    // (K <= 128: 1136 x 1968 5.2 / 5.5; nn 6.7 / 5.7) or on 256-tile problems
+    // (4096 x 4096 near even); the K-split kernel's sizes up to two workgroups
+    // a CU (256 x 512 x 512 2.9 / 4.5; past it 1024 x 1024 x 512 5.8 / 4.9, 2048
+    // x 1920 x 256 10.5 / 6.8); up to 64 tiles with K staged at once (500 x 500
+    // x 504 4.1 / 4.9, past it 800 x 800 x 512 9.0 / 4.9); and outputs of four
+    // tiles or fewer (100 x 72 x 1000 nt 6.9 / 8.2, nn 15 / 8.7).
+    const bool s32k = t32s > 0 && t32s <= 512 && (K == 256 || K == 512) && c16 && ldc % 4 == 0;
+    const bool small = K <= 64 || (K <= 128 && (bt || t256 >= 32)) || s32k ||
+                       (t64 <= 64 && K <= 512) || (t64 <= 4 && K <= 1024);
+    if (!small) {
+      // pointers only as aligned as the caller said
+      const void* al = (const void*)16;
+      const MmCall c = mm_call(al, al, (void*)16, bias ? al : nullptr, M, N, K, lda, ldb, ldc,
+                               bt, idt, odt);
+      if (mm_plan(c, &pl->mm)) {
+        pl->pipe = true;
+        snprintf(pl->name, sizeof pl->name, "%s", pl->mm.name);
+        pl->grid = (unsigned)(pl->mm.tiles_m * (long long)pl->mm.tiles_n);
+        pl->block = 256;
+        return;
+      }
+    }
     // 256 x 256 tiles (gemm_big.hip) for aligned problems from 32 tiles on:
     // one such workgroup per CU beats four 128 x 128 ones over the same
     // outputs even when most CUs stay idle (one box, fp16, K = 4096: 2048 x
     // 3072 78 against 125 us, 2560 x 4096 84 against 241; at 16 tiles the
     // smaller tiles win, 140 against 147 us); the 32-bit copy offsets of a
     // tile (up to 256 rows of A / B^T, 64 rows of B) must fit
-    const long t256 = (M % 256 == 0 && N % 256 == 0) ? (long)(M / 256) * (N / 256) : 0;
     if (t256 >= 32 && K % 64 == 0 && 256LL * lda * 2 < (1LL << 32) &&
         (bt ? 256LL : 64LL) * ldb * 2 < (1LL << 32)) {
       snprintf(pl->name, sizeof pl->name, "gemm_t256_%s_%s_%s%s", bt ? "nt" : "nn", dt, od, bs);
@@ -400,7 +436,6 @@ void gemm_plan(int M, int N, int K, int lda, int ldb, int ldc, bool bt, bool bia
       return;
     }
     const char* tile;
-    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
     int bm;
     if (t128 >= 256) { tile = "t128"; bm = 128; }
     else if (t64 >= 192) { tile = "t64"; bm = 64; }
@@ -460,6 +495,8 @@ int dense(const void* A, const void* B, void* C, const void* bias, int M, int N,
     return launch(kernel(pl.name), dim3(pl.grid), dim3(pl.block), 0, stream, A, B, C, bias, M, N,
                   K, lda, ldb, ldc, bt ? 1 : 0, idt, odt);
   }
+  if (pl.pipe)
+    return mm_launch(mm_call(A, B, C, bias, M, N, K, lda, ldb, ldc, bt, idt, odt), pl.mm, stream);
   return launch(kernel(pl.name), dim3(pl.grid), dim3(pl.block), 0, stream, A, B, C, bias, M, N,
                 K, lda, ldb, ldc);
 }
@@ -485,6 +522,9 @@ int tmhip::dense_mfma(const void* A, const void* B, void* C, int M, int N, int K
             aligned16(C), &pl);
   if (pl.general) return 0;
   *used = true;
+  if (pl.pipe)
+    return mm_launch(mm_call(A, B, C, nullptr, M, N, K, lda, ldb, ldc, bt, in_dtype, out_dtype),
+                     pl.mm, stream);
   return launch(kernel(pl.name), dim3(pl.grid), dim3(pl.block), 0, stream, A, B, C,
                 (const void*)nullptr, M, N, K, lda, ldb, ldc);
 }

@@ -113,6 +113,30 @@ int dense_f32(const float* A, const float* B, void* C, int M, int N, int K, int 
 int dense_mfma(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb,
                int ldc, bool bt, int in_dtype, int out_dtype, void* stream, bool* used);
 
+// One product of the pipelined MFMA kernels (ops_mm.cpp, gemm_pipe.h):
+// C[b, m, n] = sum_k A[b, m, k] B[b, k, n] (+ Z[b, m, n], Z null for none; a
+// row or column Z has a zero stride along the other dimension), strides in
+// elements.
+struct MmCall {
+  const void* A;
+  const void* B;
+  const void* Z;
+  void* C;
+  int batch, M, N, K;
+  long long sa_b, sa_m, sa_k, sb_b, sb_k, sb_n, sc_b, sc_m, sc_n, sz_b, sz_m, sz_n;
+  int in_dt, out_dt, z_dt;
+};
+struct MmPlan {
+  char name[32];
+  const char* tile;
+  int tiles_m, tiles_n;
+  bool arc, brc;  // operand row-contiguous (else k-contiguous)
+};
+// The kernel for a call (pointers only inspected for their alignment), or
+// false when these kernels do not take it; then its launch.
+bool mm_plan(const MmCall& c, MmPlan* pl);
+int mm_launch(const MmCall& c, const MmPlan& pl, void* stream);
+
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 inline bool is_half(int dt) { return dt == TM_DT_F16 || dt == TM_DT_BF16; }
 inline bool is_float(int dt) { return dt == TM_DT_F32 || dt == TM_DT_F16 || dt == TM_DT_BF16; }
