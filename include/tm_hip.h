@@ -332,6 +332,10 @@ int tm_flash_attention(const void* q, const void* k, const void* v, void* o, flo
  * query elements beyond that saturate at +-131008. */
 size_t tm_decode_attention_workspace_size(int batch, int q_heads, int kv_heads, int head_dim,
                                           int seq_len, int page_size);
+/* The workspace with which 16-bit caches take the slices that fill the device
+ * best (a smaller one: as above); never less than the size above. */
+size_t tm_decode_attention_full_workspace_size(int batch, int q_heads, int kv_heads,
+                                               int head_dim, int seq_len, int page_size);
 int tm_decode_attention(const void* q, const void* k_cache, const void* v_cache, void* o,
                         float* lse, int batch, int q_heads, int kv_heads, int head_dim,
                         const int* seq_lens, int seq_len, const long long* kv_strides,

@@ -300,3 +300,35 @@ def test_decode_fp32_query_beyond_fp16_range(dev):
     assert np.isfinite(got).all()
     np.testing.assert_allclose(got, ref, atol=1e-4, rtol=1e-4)
     np.testing.assert_allclose(lse.cpu().numpy(), ref_l, atol=1e-4, rtol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("page_size,S", [(1, 130), (5, 700), (16, 2100), (24, 1600)])
+def test_paged_slices_past_64_pages(page_size, S):
+    """Enough sequences x heads that a slice is a whole sequence of more than 64
+    pages (the page ids are reloaded every 64 pages), lengths on both sides of
+    those boundaries, page ids past the table's used part never read."""
+    B, Hkv, rep, D = 96, 8, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(page_size)
+    per = -(-S // page_size)
+    q = torch.randn(B, Hkv * rep, D, device="cuda", generator=g).half()
+    kc, vc = (torch.randn(2 * per, page_size, Hkv, D, device="cuda", generator=g).half()
+              for _ in range(2))
+    edges = [1, 32, 64 * page_size - 1, 64 * page_size, 64 * page_size + 1, 65 * page_size, S]
+    lens = [min(S, edges[i % len(edges)]) for i in range(B)]
+    table = torch.randint(0, 2 * per, (B, per), device="cuda", generator=g, dtype=torch.int32)
+    for b, n in enumerate(lens):
+        table[b, -(-n // page_size):] = 1 << 30  # unused entries
+    o = tm.decode_attention(q, kc, vc, seq_lens=torch.tensor(lens, dtype=torch.int32,
+                                                             device="cuda"),
+                            seq_len=S, page_table=table)
+    for b in list(range(2 * len(edges))) + [B - 1]:
+        n = lens[b]
+        used = table[b, :-(-n // page_size)].long()
+        k, v = (t[used].reshape(-1, Hkv, D)[:n].transpose(0, 1).float() for t in (kc, vc))
+        qf = q[b].float().reshape(Hkv, rep, D)
+        p = torch.softmax((qf.unsqueeze(2) * k.unsqueeze(1)).sum(-1) * D ** -0.5, -1)
+        ref = (p.unsqueeze(-1) * v.unsqueeze(1)).sum(2).reshape(Hkv * rep, D)
+        # P and O round to fp16: 2^-11 of the weighted sum of |V| each
+        tol = 2.0 ** -10 * (p.unsqueeze(-1) * v.abs().unsqueeze(1)).sum(2).reshape(ref.shape)
+        assert bool(((o[b].float() - ref).abs() <= tol + 1e-4).all()), (b, n)

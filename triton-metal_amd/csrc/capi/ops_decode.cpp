@@ -3,6 +3,7 @@
 // 48 / 80 / 96 / 112, decode_attn_d<64|128>v<D>_<dt> (16-bit caches) or
 // decode_attn_f32_d<D> (fp32), + decode_attn_combine when the sequence is
 // split into slices, or decode_attn_general.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -35,7 +36,15 @@ struct DecodeParams {
 
 bool is16(int dt) { return dt == TM_DT_F16 || dt == TM_DT_BF16; }
 
-// Slices of the positions for the MFMA kernel: about one resident round of
+// Granularity of a slice: 32 positions, and whole pages.
+int slice_unit(int page_size, bool paged) {
+  if (!paged) return 32;
+  int g = 32, r = page_size;  // lcm(page_size, 32)
+  while (r) { const int t = g % r; g = r; r = t; }
+  return page_size / g * 32;
+}
+
+// Slices of the positions for the MFMA kernels: about one resident round of
 // waves (B * kv_heads * head blocks * slices ~ 768: three 48 KB rings per CU)
 // with at least 256 positions per slice, a multiple of 32 (and, paged, whole
 // pages, at most 64 of them).
@@ -47,9 +56,7 @@ void plan_split(int batch, int q_heads, int kv_heads, int cap, int page_size, bo
   int sl = std::max(256, (cap + want - 1) / want);
   sl = (sl + 31) / 32 * 32;
   if (paged) {
-    int g = 32, r = page_size;  // unit = lcm(page_size, 32)
-    while (r) { const int t = g % r; g = r; r = t; }
-    const int unit = page_size / g * 32;
+    const int unit = slice_unit(page_size, paged);
     sl = (sl + unit - 1) / unit * unit;
     const long long maxsl = 64LL * page_size / 32 * 32;  // 64 pages, whole tiles
     if (sl > maxsl) sl = (int)(maxsl / unit * unit);
@@ -57,6 +64,37 @@ void plan_split(int batch, int q_heads, int kv_heads, int cap, int page_size, bo
   if (sl <= 0) sl = 32;
   *split_len = sl;
   *nsplit = (cap + sl - 1) / sl;
+}
+
+// Slices for the 16-bit kernels when the workspace has room for them
+// (tm_decode_attention_full_workspace_size): of any number of pages, their
+// number the one whose rounds of resident waves (160 KB of LDS per CU over the
+// ring of a wave) take least.  In positions of a wave's time: 100 for its
+// start, 75 for the combining launch and more past the 32 slices that it
+// merges at once.  Against the plan above (us, fp16, 16-position pages unless
+// said): 16 sequences of 2.5 to 8 k positions, 8 KV heads 146 -> 103 (8 slices
+// of 64 pages put 1024 waves on 768 places); 64 sequences of up to 1000, 64-
+// position pages 75 -> 60; 3 sequences of up to 2314, D = 96 23 -> 15 (9 slices left
+// most places empty).
+void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, int page_size,
+                 bool paged, int* nsplit, int* split_len) {
+  const int group = q_heads / kv_heads, hbn = (group + 15) / 16;
+  const long long segs = (long long)batch * kv_heads * hbn;
+  const long long slots = 256LL * (head_dim <= 64 ? 6 : 3);
+  const int unit = slice_unit(page_size, paged);
+  double best = 0;
+  *nsplit = 0;
+  for (int n = 1; n <= 256; ++n) {
+    long long sl = (cap + n - 1) / n;
+    sl = (sl + unit - 1) / unit * unit;
+    if (n > 1 && sl < 64) break;
+    const double cost = (double)((segs * n + slots - 1) / slots) * (double)(sl + 100) +
+                        (n > 1 ? 75 + 2 * std::max(0, n - 32) : 0);
+    if (*nsplit && cost >= best) continue;
+    best = cost;
+    *nsplit = (int)((cap + sl - 1) / sl);
+    *split_len = (int)sl;
+  }
 }
 
 }  // namespace
@@ -70,6 +108,21 @@ extern "C" size_t tm_decode_attention_workspace_size(int batch, int q_heads, int
   plan_split(batch, q_heads, kv_heads, seq_len, page_size > 0 ? page_size : 1, page_size > 0,
              &ns, &sl);
   return ns > 1 ? (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float) : 0;
+}
+
+extern "C" size_t tm_decode_attention_full_workspace_size(int batch, int q_heads, int kv_heads,
+                                                          int head_dim, int seq_len,
+                                                          int page_size) {
+  const size_t base = tm_decode_attention_workspace_size(batch, q_heads, kv_heads, head_dim,
+                                                         seq_len, page_size);
+  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || head_dim <= 0 ||
+      seq_len <= 0)
+    return 0;
+  int ns = 1, sl = 0;
+  plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, page_size > 0 ? page_size : 1,
+              page_size > 0, &ns, &sl);
+  return std::max(base, ns > 1 ? (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float)
+                               : (size_t)0);
 }
 
 // Both entry points.  noalloc: the slice partials go to the device's
@@ -139,6 +192,11 @@ static int decode_attention(const char* op, bool noalloc, const void* q, const v
   if (mfma) {
     int ns = 1, sl = 0;
     plan_split(batch, q_heads, kv_heads, seq_len, p.page_size, paged, &ns, &sl);
+    if (!f32 && !noalloc && workspace && aligned16(workspace) &&
+        workspace_bytes >= tm_decode_attention_full_workspace_size(
+                               batch, q_heads, kv_heads, head_dim, seq_len,
+                               paged ? page_size : 0))
+      plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged, &ns, &sl);
     const size_t need = (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float);
     if (noalloc && ns > 1) {
       static DeviceGlobal scratch("tm_decode_scratch");

@@ -50,7 +50,7 @@ struct DecodeParams {
   int page_size, max_pages;
   int page_shift;           // log2(page_size) when a power of two, else -1
   int nsplit, split_len;    // slices of split_len positions (paged: whole
-                            // pages, at most 64 of them)
+                            // pages; fp32 caches at most 64 of them)
   float sl2;                // scale * log2(e)
   int q_dt, kv_dt, o_dt;    // TM_DT_* codes
 };
@@ -175,18 +175,24 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeParams& p) {
   const int* pt = p.page_table ? p.page_table + (long long)b * p.max_pages : nullptr;
   const uint32_t lbase = __builtin_amdgcn_readfirstlane(lds_off(lds));
   const int ntile = p1 > p0 ? (p1 - p0 + 31) / 32 : 0;
-  // paged: lane i holds the physical page of the slice's i-th page (the slice
-  // starts on a page boundary and spans at most 64 pages), fetched below with
-  // ds_bpermute so that no table load sits between the copies
-  const int fp = pt ? p0 / p.page_size : 0;
-  int mypage = 0;
-  if (pt && ntile > 0) {
-    const int np = (p1 - 1) / p.page_size - fp + 1;
-    if (lane < np) mypage = pt[fp + lane];
-  }
+  // paged: the slice starts on a page boundary; lane i holds the physical page
+  // of the i-th page of the current 64 pages (whole 32-position tiles), fetched
+  // below with ds_bpermute so that no table load sits between the copies, and
+  // loaded anew at every 64th page
+  const int fp = pt ? p0 / p.page_size : 0, np = pt && ntile > 0 ? (p1 - 1) / p.page_size - fp + 1 : 0;
+  int mypage = lane < np ? pt[fp + lane] : 0;
+  int pb0 = p0, reload = 2 * p.page_size;  // first position; tile of the next 64 pages
+  auto next_pages = [&](int t) {
+    if (pt && t == reload) {
+      const int i = 32 * t / p.page_size + lane;
+      mypage = i < np ? pt[fp + i] : 0;
+      pb0 = p0 + 32 * t;
+      reload += 2 * p.page_size;
+    }
+  };
   auto row_off = [&](int pos) -> long long {  // element offset of cache position pos
     if (pt) {
-      const int rel = pos - p0;  // p0 is page aligned
+      const int rel = pos - pb0;  // pb0 is page aligned
       const int pi = p.page_shift >= 0 ? rel >> p.page_shift : rel / p.page_size;
       const int slot = p.page_shift >= 0 ? rel & (p.page_size - 1) : rel - pi * p.page_size;
       const int page = __builtin_amdgcn_ds_bpermute(4 * pi, mypage);
@@ -213,6 +219,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeParams& p) {
     }
   }
   auto issue = [&](int t) {
+    next_pages(t);
     const uint32_t st = lbase + (uint32_t)((t % NST) * 2 * TB);
     // all row offsets first (paged: the page fetches overlap), then the copies
     long long e[NCP];

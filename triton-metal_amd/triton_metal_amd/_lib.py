@@ -67,6 +67,7 @@ SIGNATURES = {
                            C.c_float, i32, i32, vp],
     "tm_kda_workspace_size": [i32, i32, i32, i32, i32, i32],
     "tm_decode_attention_workspace_size": [i32, i32, i32, i32, i32, i32],
+    "tm_decode_attention_full_workspace_size": [i32, i32, i32, i32, i32, i32],
     "tm_decode_attention": [vp, vp, vp, vp, vp, i32, i32, i32, i32, vp, i32,
                             C.POINTER(C.c_longlong), vp, i32, i32, C.c_float, i32, i32, i32, vp,
                             sz, vp],
@@ -84,6 +85,7 @@ _RESTYPES = {
     "tm_builtin_module_name": C.c_char_p,
     "tm_kda_workspace_size": sz,
     "tm_decode_attention_workspace_size": sz,
+    "tm_decode_attention_full_workspace_size": sz,
     "tm_wq_workspace_bytes": sz,
 }
 

@@ -839,8 +839,8 @@ def plan_decode_attention(q, k_cache, v_cache, o, seq_lens=None, seq_len=None, p
         raise ValueError("lse must be fp32 [B, Hq]")
     if scale is None:
         scale = D ** -0.5
-    need = _lib.lib().tm_decode_attention_workspace_size(B, Hq, Hkv, D, seq_len,
-                                                         page_size if page_table is not None else 0)
+    need = _lib.lib().tm_decode_attention_full_workspace_size(
+        B, Hq, Hkv, D, seq_len, page_size if page_table is not None else 0)
     if workspace is None and need > 0:
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     wbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
