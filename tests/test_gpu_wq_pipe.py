@@ -1,0 +1,79 @@
+"""The pipelined weight-only kernels (wq_pipe.hip): edges of their tiles and k
+slices against the fp32 product, and the calls that select them."""
+import pytest
+import torch
+
+import triton_metal_amd as tm
+
+ACT = {"f16": torch.float16, "bf16": torch.bfloat16}
+
+
+def _problem(qbits, M, N, K, act, zeros, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(M, K, generator=g).to(act)
+    cols = K // 128 if qbits == 4 else 1
+    if qbits == 4:
+        w = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8)
+        q = torch.stack((w & 15, w >> 4), -1).reshape(N, K).double()
+    else:
+        w = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8)
+        q = w.double()
+    s = ((0.5 + torch.rand(N, cols, generator=g)) / 64).to(act)
+    z = None
+    if zeros == "u":
+        z = torch.randint(0, 256, (N, cols), generator=g).to(torch.uint8)
+    elif zeros == "s":  # fractional zero-points too
+        z = (torch.rand(N, cols, generator=g) * 15).to(act)
+    rep = K // cols
+    deq = s.double().repeat_interleave(rep, 1)
+    mag = (q.abs() + (0 if z is None else z.double().repeat_interleave(rep, 1)) +
+           (1024 if qbits == 4 else 0)) * deq
+    deq = deq * (q - (0 if z is None else z.double().repeat_interleave(rep, 1)))
+    return x, w, s if qbits == 4 else s.reshape(N), z, deq, mag
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ACT)
+@pytest.mark.parametrize("qbits,zeros", [(4, None), (4, "s"), (4, "u"), (8, None)])
+@pytest.mark.parametrize("M,N,K", [(1, 144, 640), (2, 48, 128), (13, 272, 1152), (64, 128, 384),
+                                   (65, 400, 896), (129, 16, 2176), (200, 1040, 3200),
+                                   (1300, 2064, 384)])
+def test_against_the_fp32_product(qbits, zeros, act, M, N, K):
+    dt = ACT[act]
+    x, w, s, z, deq, mag = _problem(qbits, M, N, K, dt, zeros, M + N)
+    if not (qbits == 4 and M == 1):
+        name = tm.wq_kernel_for(qbits, M, N, K, act_dtype=dt, details=True, zero_dtype=None if z is
+                                None else z.dtype)["name"]
+        assert name == f"wq_pipe_q{qbits}_{act}_z{zeros or 'n'}_r{1 if M <= 64 else 2}", name
+    bias = torch.randn(N).to(dt)
+    xd, wd, sd, bd = x.cuda(), w.cuda(), s.cuda(), bias.cuda()
+    zd = None if z is None else z.cuda()
+    y = torch.full((M, N), float("nan"), dtype=dt, device="cuda")
+    if qbits == 4:
+        tm.int4_linear(xd, wd, bd, y, sd, zd, M, N, K, 128)
+    else:
+        tm.int8_linear(xd, wd, bd, y, sd, zd, M, N, K)
+    ref = x.double() @ deq.t() + bias.double()
+    # one rounding of the result, and fp32 sums of OFF + q and z sum x
+    u = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    tol = 1.01 * u * ref.abs() + 2.0 ** -24 * (K ** 0.5 * 4) * (x.double().abs() @ mag.t()) + 1e-6
+    err = (y.cpu().double() - ref).abs()
+    assert bool((err <= tol).all()), float((err / tol).max())
+
+
+def test_selection():
+    """Sizes on both sides of the pipelined kernels' rules (no device is touched)."""
+    k = lambda *a, **kw: tm.wq_kernel_for(*a, **kw, details=True)
+    f16, bf16, u8 = torch.float16, torch.bfloat16, torch.uint8
+    assert k(4, 228, 2816, 7040, act_dtype=bf16)["name"] == "wq_pipe_q4_bf16_zn_r2"
+    assert k(4, 1000, 4096, 11008, zero_dtype=u8)["name"] == "wq_pipe_q4_f16_zu_r2"
+    assert k(4, 1000, 4096, 4096, zero_dtype=u8)["name"].startswith("wq_wide_")
+    assert k(8, 11, 1280, 3456)["name"] == "wq_pipe_q8_f16_zn_r1"
+    # without the workspace int4 stays where it was
+    assert k(4, 228, 2816, 7040, with_workspace=False)["name"] == "wq_general"
+    assert k(8, 700, 22016, 4096, with_workspace=False)["workspace_bytes"] == 0
+    d = k(4, 8, 1280, 3712)
+    assert d["splits"] > 1 and d["workspace_bytes"] >= d["splits"] * 8 * 1280 * 4 + 8 * 3712 * 2
+    # zero-points of int8, and groups other than 128, are not theirs
+    assert not k(8, 11, 1280, 3456, zero_dtype=f16)["name"].startswith("wq_pipe")
+    assert not k(4, 11, 1280, 3456, 64)["name"].startswith("wq_pipe")

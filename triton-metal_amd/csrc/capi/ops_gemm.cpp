@@ -34,7 +34,7 @@ Kernel& kernel(const std::string& name) { return tmhip::kernel_named(name); }
 // form of a kernel over `splits` k-slices, grid (grid, splits), writing fp32
 // [splits][M][N] into the workspace, then wq_splitk_reduce_<act>.
 enum { WQ_ARGS_STD = 0, WQ_ARGS_G = 1, WQ_ARGS_GENERAL = 2, WQ_ARGS_SPLIT = 3,
-       WQ_ARGS_SPLIT_G = 4 };
+       WQ_ARGS_SPLIT_G = 4, WQ_ARGS_PIPE = 5 };
 struct WqPlan {
   char name[64];
   unsigned grid, block, lds;
@@ -42,6 +42,33 @@ struct WqPlan {
   int splits;     // k-slices (1: no split)
   int kslice;     // k per slice (the last may be shorter: WQ_ARGS_SPLIT_G)
   size_t ws;      // workspace bytes (split-K plans)
+};
+
+// Workspace of a wq_pipe plan: the permuted X and the group sums (int4), then
+// the fp32 slice sums; kernel arguments (struct WqPipeParams of wq_pipe.hip).
+struct WqPipeWs {
+  size_t sx, p, total;
+  int sxld;
+};
+WqPipeWs wq_pipe_ws(int qbits, int M, int N, int K, int splits) {
+  WqPipeWs w;
+  w.sxld = (M + 3) & ~3;
+  w.sx = qbits == 4 ? ((size_t)M * K * 2 + 255) & ~(size_t)255 : 0;
+  w.p = qbits == 4 ? w.sx + (((size_t)(K / 128) * w.sxld * 4 + 255) & ~(size_t)255) : 0;
+  w.total = w.p + (splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0);
+  return w;
+}
+struct WqPipeParams {
+  const void* X;
+  const void* W;
+  const void* S;
+  const void* Z;
+  const float* SX;
+  void* Y;
+  float* P;
+  const void* bias;
+  int M, N, K, kslice;
+  int tiles_m, tiles_n, sxld;
 };
 
 void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, unsigned align,
@@ -63,6 +90,41 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
                     (qbits == 8 || G % 128 == 0) && N % 16 == 0 && K > 0 && a16;
   const char* act = adt == TM_DT_BF16 ? "bf16" : "f16";
   const char zc = zdt == TM_DT_NONE ? 'n' : (zdt == TM_DT_U8 ? 'u' : 's');
+  // pipelined tiles (wq_pipe.hip): int4 with groups of 128 (which needs the
+  // workspace for its copy of X), int8 without zero-points
+  const bool pipe_ok = fast && K % 128 == 0 && (long long)K * 256 < (1LL << 31) &&
+                       (qbits == 4 ? G == 128 && split_ok : zdt == TM_DT_NONE);
+  auto pipe = [&]() {
+    const int rt = M <= 64 ? 1 : 2;
+    const int tm = (M + 64 * rt - 1) / (64 * rt), tn = (N + 127) / 128, groups = K / 128;
+    // k slices for about two workgroups per CU, at least four groups each
+    int S = 1, per = groups;
+    if (split_ok && (long)tm * tn < 2 * cus) {
+      const int want = (int)std::max<long>(
+          1, std::min<long>(std::min(16, groups / 4), 2L * cus / ((long)tm * tn)));
+      per = (groups + want - 1) / want;
+      S = (groups + per - 1) / per;
+    }
+    snprintf(pl->name, sizeof pl->name, "wq_pipe_q%d_%s_z%c_r%d", qbits, act, zc, rt);
+    set((unsigned)(tm * tn), 256, 0, WQ_ARGS_PIPE);
+    pl->splits = S;
+    pl->kslice = per * 128;
+    pl->ws = wq_pipe_ws(qbits, M, N, K, S).total;
+  };
+  // wide kernel (below): K in steps it can walk and aligned scales
+  const bool w4k = qbits == 4 && (K % 512 == 0 || (K % 256 == 0 && zdt != TM_DT_U8));
+  const bool wide = fast && M > 64 && N % 128 == 0 && s16 && z16 &&
+                    ((w4k && adt == TM_DT_F16 && G == 128) ||
+                     (qbits == 8 && zdt == TM_DT_NONE && K % 128 == 0));
+  // Products of enough 128 x 128 tiles: 160 against the tiled and streaming
+  // kernels and the wide kernel's split form (us, M = 1000: fp16 u8 zero-points
+  // K = 11008 N = 4096 239 -> 128; bf16 K = 4096 N = 4096 90 -> 58, N = 28672
+  // 593 -> 277), more against the wide kernel in one launch (fp16 K = 4096: 256
+  // tiles 50 here 60, 392 109 here 88, 768 144 here 129; int8 M = 700: 240 tiles
+  // 38 here 42, 288 63 here 56, 1032 167 here 153)
+  const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+  if (pipe_ok && M > 64 && t128 >= (!wide || (qbits == 4 && K > 4096) ? 160 : qbits == 4 ? 320 : 280))
+    return pipe();
   // wide kernel: M > 64, 64 x 128 output blocks (int4: fp16 activations;
   // int8: fp16 or bf16).  With a workspace, split-K over S k-slices when its
   // tiles would fill less than half the CUs, or when int4 K exceeds the 4096
@@ -70,10 +132,7 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
   // (int4: K % 512 == 0 with uint8 zero-points, whose per-row bytes the
   // split form gathers as dwords; K % 256 == 0 otherwise.  Where no equal
   // slicing fits, slices of whole units with a shorter last one.)
-  const bool w4k = qbits == 4 && (K % 512 == 0 || (K % 256 == 0 && zdt != TM_DT_U8));
-  if (fast && M > 64 && N % 128 == 0 && s16 && z16 &&
-      ((w4k && adt == TM_DT_F16 && G == 128) ||
-       (qbits == 8 && zdt == TM_DT_NONE && K % 128 == 0))) {
+  if (wide) {
     const int ns = qbits == 4 ? 3 : 4, ck = qbits == 4 ? 64 : 32;
     const int unit = qbits == 4 ? (K % 512 == 0 ? 512 : 256) : 128;  // slice granularity
     const int mtl = (M + 63) / 64, ntl = N / 128;
@@ -250,6 +309,15 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
     snprintf(pl->name, sizeof pl->name, "wq_skinny_q%d_%s_z%c%s", qbits, act, zc, vs ? "_v" : "");
     return set(N / 16, 256, lds, WQ_ARGS_G);
   }
+  // K no multiple of 256 or N of 64 would run on wq_general (us, int4: M = 228
+  // K = 7040 N = 2816 1367 -> 30, M = 100 K = 9600 N = 4096 830 -> 31, M = 8 K =
+  // 3712 N = 1280 23 -> 14; int8 M = 11 K = 3456 31 -> 12).  K of at most 4096
+  // that is a multiple of 256 only: larger weights (M = 3 K = 3840 N = 11520 28
+  // -> 19, N = 3840 12 here 13; M = 228 K = 2816 N = 2816 26 -> 23, M = 28 K =
+  // 1280 N = 1920 14 here 16: the permuting launch and the reduction cost 4)
+  if (pipe_ok && (K % 256 != 0 || N % 64 != 0 ||
+                  (K <= 4096 && M > 1 && (long long)N * K >= (M > 64 ? 5000000 : 20000000))))
+    return pipe();
   // tiled kernel: 64 x 64 output tiles walking K in steps of 256.  With a
   // workspace and fewer tiles than CUs: split-K over slices of whole steps
   // (the last one shorter), about two workgroups per CU, at most 16 slices
@@ -314,6 +382,35 @@ int wq_matmul(int qbits, const void* X, const void* W, void* Y, const void* S, c
   Kernel& k = kernel(pl.name);
   const dim3 grid(pl.grid), block(pl.block);
   switch (pl.form) {
+    case WQ_ARGS_PIPE: {
+      const WqPipeWs w = wq_pipe_ws(qbits, M, N, K, pl.splits);
+      if (w.total > workspace_bytes)
+        return fail(TM_ERR_INVALID_ARG, "%s: workspace of %zu bytes, this call needs %zu", op,
+                    workspace_bytes, w.total);
+      char* ws = (char*)workspace;
+      WqPipeParams p;
+      memset(&p, 0, sizeof p);
+      p.X = X; p.W = W; p.S = S; p.Z = Z; p.Y = Y; p.bias = bias;
+      p.M = M; p.N = N; p.K = K; p.kslice = pl.kslice; p.sxld = w.sxld;
+      p.tiles_n = (N + 127) / 128;
+      p.tiles_m = (int)pl.grid / p.tiles_n;
+      if (qbits == 4) {
+        p.X = ws;
+        p.SX = (const float*)(ws + w.sx);
+        const int rc = launch(
+            kernel(adt == TM_DT_BF16 ? "wq_pipe_prep_bf16" : "wq_pipe_prep_f16"),
+            dim3((unsigned)((K + 2047) / 2048), (unsigned)M), dim3(256), 0, stream, X, (void*)ws,
+            (void*)(ws + w.sx), K, w.sxld);
+        if (rc) return rc;
+      }
+      p.P = pl.splits > 1 ? (float*)(ws + w.p) : nullptr;
+      int rc = launch(k, dim3(pl.grid, (unsigned)pl.splits), block, 0, stream, p);
+      if (rc || pl.splits == 1) return rc;
+      const size_t quads = (size_t)M * N / 4;
+      return launch(kernel(adt == TM_DT_BF16 ? "wq_splitk_reduce_bf16" : "wq_splitk_reduce_f16"),
+                    dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream,
+                    (const float*)p.P, Y, bias, M, N, pl.splits);
+    }
     case WQ_ARGS_SPLIT:
     case WQ_ARGS_SPLIT_G: {
       float* P = (float*)workspace;

@@ -44,7 +44,9 @@ HIPCC_FLAGS = [
 # compiler's choice for kda_state, whose state update scales and packs every
 # result on the VALU, would move each one out of AGPRs and back every chunk;
 # the file's other kernels compile identically either way).
+# wq_pipe.hip: the same for its group sums, which the VALU scales and adds.
 EXTRA_FLAGS = {
+    "wq_pipe": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kda": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
