@@ -340,3 +340,22 @@ def test_kda_graph_replays_track_new_inputs(dev):
         assert torch.equal(o, o_ref), f"replay with inputs {seed}: o"
         assert torch.equal(st, st_ref), f"replay with inputs {seed}: final state"
     del graph
+
+
+@pytest.mark.gpu
+def test_kda_segments_match_separate_calls():
+    """Enough chunks that one call walks the sequence in segments (1846 chunks:
+    two of 36 and 35 chunks a head, the last one partial): the same bits as two
+    calls cut elsewhere with the state handed over."""
+    B, T, H = 2, 64 * 70 + 5, 13
+    q, k, v, g, beta = (t.cuda() for t in kda_inputs(B, T, H, seed=9))
+    s0 = 0.1 * torch.randn(B, H, 128, 128, generator=torch.Generator().manual_seed(1)).cuda()
+    o, st = tm.chunk_kda(q, k, v, g, beta, initial_state=s0, output_final_state=True)
+    o_only, none = tm.chunk_kda(q, k, v, g, beta, initial_state=s0)
+    cut = 64 * 50
+    first, rest = ([t[:, :cut].contiguous() for t in (q, k, v, g, beta)],
+                   [t[:, cut:].contiguous() for t in (q, k, v, g, beta)])
+    o1, mid = tm.chunk_kda(*first, initial_state=s0, output_final_state=True)
+    o2, end = tm.chunk_kda(*rest, initial_state=mid, output_final_state=True)
+    assert none is None and torch.equal(o, o_only)
+    assert torch.equal(o, torch.cat((o1, o2), 1)) and torch.equal(st, end)

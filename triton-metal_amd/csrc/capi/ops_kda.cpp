@@ -102,16 +102,36 @@ extern "C" int tm_kda_chunk_fwd(const void* q, const void* k, const void* v, con
   p.scale = scale;
   p.beta_bf16 = beta_dtype == TM_DT_BF16 ? 1 : 0;
 
-  if (nc > 0) {
-    // two workgroups per CU (their LDS and registers admit no third), each
-    // walking its share of the chunks
-    p.c0 = 0; p.c1 = (int)nc;
-    const long long grid = std::min<long long>(bh * nc, 2LL * cu_count());
-    const int rc = launch(intra_kernel(), dim3((unsigned)grid), dim3(256), 0, stream, p);
-    if (rc) return rc;
+  // A workspace past half of the 256 MB Infinity Cache is written by kda_intra
+  // and read back by kda_state from HBM, and each call evicts the last one's.
+  // So from 1536 chunks (114 MB) the sequence goes through the two kernels in
+  // segments of at most 1200 chunks (89 MB) that share one place, the state
+  // handed over in fp32 behind it.  us per call, three calls' buffers in turn:
+  // B = 1, H = 16, T = 8192 (2048 chunks) 236 -> 183; H = 32, T = 4300 (2176)
+  // 181 -> 168 (24 to 48 chunks a segment: 172, 159); below the line it only
+  // adds launches: H = 8, T = 8000 (1000) 127 -> 138 in two segments.  A
+  // sequence of fewer than 64 chunks is not cut (B = 3, H = 20, 32 chunks each:
+  // 219 -> 228 in two).
+  const long long nseg = bh * nc > 1536 && nc >= 64 ? (bh * nc + 1199) / 1200 : 1;
+  const int seg = (int)std::max<long long>(nseg > 1 ? 16 : 0, (nc + nseg - 1) / nseg);
+  float* hand = (float*)((char*)workspace + (size_t)bh * seg * kChunkBytes);
+  p.NC = seg;
+  for (int c0 = 0;; c0 += seg) {
+    p.c0 = c0;
+    p.c1 = (int)std::min<long long>(nc, c0 + seg);
+    p.st = p.c1 < nc ? hand : final_state;
+    if (p.c1 > c0) {
+      // two workgroups per CU (their LDS and registers admit no third), each
+      // walking its share of the chunks
+      const long long grid = std::min<long long>(bh * (p.c1 - c0), 2LL * cu_count());
+      const int rc = launch(intra_kernel(), dim3((unsigned)grid), dim3(256), 0, stream, p);
+      if (rc) return rc;
+    }
+    const int rc = launch(state_kernel(), dim3((unsigned)(bh * (kValueDim / 16))), dim3(192), 0,
+                          stream, p);
+    if (rc || p.c1 >= nc) return rc;
+    p.s0 = hand;
   }
-  p.c0 = 0; p.c1 = (int)nc;
-  return launch(state_kernel(), dim3((unsigned)(bh * (kValueDim / 16))), dim3(192), 0, stream, p);
 }
 
 extern "C" int tm_kda_recurrent_fwd(const void* q, const void* k, const void* v, const float* g,

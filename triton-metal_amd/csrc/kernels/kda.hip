@@ -105,8 +105,8 @@ struct KdaParams {
   const float* s0;     // [B, H, KD, VD] fp32 or null
   uint16_t* o;         // [B, T, H, VD] bf16
   float* st;           // [B, H, KD, VD] fp32 or null
-  uint8_t* ws;         // workspace: B*H*NC chunks of WS_CHUNK bytes
-  int B, T, H, NC;
+  uint8_t* ws;         // workspace: NC chunks of WS_CHUNK bytes per (batch, head)
+  int B, T, H, NC;     // (the chunks of one launch: chunk c in place c - c0)
   int c0, c1;          // the chunks [c0, c1) of every (batch, head) this launch covers
   float scale;
   int beta_bf16;
@@ -176,14 +176,14 @@ void kda_intra(KdaParams p) {
   const int total = p.B * p.H * nsc;
 
   struct Chunk {
-    int gidx;  // workspace chunk index bh * NC + chunk
+    int gidx;  // workspace chunk index bh * NC + chunk - c0
     int b, h, t0, nt;
     long long base_k, base_v;
   };
   auto locate = [&](int idx) {
     Chunk c;
     const int bh = idx / nsc, chunk = p.c0 + (idx - bh * nsc);
-    c.gidx = bh * p.NC + chunk;
+    c.gidx = bh * p.NC + chunk - p.c0;
     c.b = bh / p.H;
     c.h = bh - c.b * p.H;
     c.t0 = chunk * KC;
@@ -576,7 +576,7 @@ extern "C" __global__ __launch_bounds__(192) void kda_state(KdaParams p) {
   const int v0 = vs * 16;
   const long long rsv = (long long)p.H * VD;
   const uint8_t* wsh = p.ws + (size_t)bh * p.NC * WS_CHUNK;
-  auto chunk_ws = [&](int c) { return wsh + (size_t)min(c, p.c1 - 1) * WS_CHUNK; };
+  auto chunk_ws = [&](int c) { return wsh + (size_t)(min(c, p.c1 - 1) - p.c0) * WS_CHUNK; };
 
   if (wave == 0) {
     // ---- the recurrence --------------------------------------------------
