@@ -22,7 +22,7 @@ class Params(ctypes.Structure):
                 + [(n, ctypes.c_longlong) for n in ("sa_b", "sb_b", "sc_b", "sz_b", "sc_m",
                                                     "sc_n", "sz_m", "sz_n")]
                 + [(n, ctypes.c_int) for n in ("M", "N", "K", "lda", "ldb", "tiles_m", "tiles_n",
-                                               "epi", "out_dt", "z_dt", "vec_z")])
+                                               "epi", "out_dt", "z_dt", "vec_z", "fix")])
 
 
 def _operand(b, rows, cols, dt, transposed, seed, al):
@@ -93,6 +93,33 @@ def test_every_kernel(kind, layout, tile):
         torch.cuda.synchronize()
         # the fp32 sum and the addition of Z each round once more
         _close(C, ref, bound + 2 * U[torch.float32] * ref.abs(), odt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", KINDS.values(), ids=KINDS)
+@pytest.mark.parametrize("M,N,K", [(5, 70, 33), (129, 257, 131), (64, 33, 1), (300, 190, 1027),
+                                   (131, 515, 575), (1, 1, 200)])
+def test_any_alignment(dt, M, N, K):
+    """Operands that start anywhere, with any row length and any K, in every
+    layout; NaN around them (and in the row after the one a piece crosses into)
+    never reaches the result."""
+    for ta in (False, True):
+        for tb in (False, True):
+            for off, pad in ((0, 0), (1, 3), (3, 1)):
+                def place(rows, cols, seed):
+                    g = torch.Generator().manual_seed(seed)
+                    flat = torch.full((off + rows * (cols + pad),), float("nan")).to(dt)
+                    t = flat[off:].view(rows, cols + pad)
+                    t[:, :cols] = torch.randn(rows, cols, generator=g).to(dt)
+                    return flat.cuda()[off:].view(rows, cols + pad)[:, :cols]
+                a = place(K, M, 1).t() if ta else place(M, K, 1)
+                b = place(N, K, 2).t() if tb else place(K, N, 2)
+                c = torch.full((M, N), 7.0, device="cuda")
+                tm.dot(a, b, c)
+                torch.cuda.synchronize()
+                ref = a.double() @ b.double().contiguous()
+                bound = K * U[torch.float32] * (a.double().abs() @ b.double().abs().contiguous())
+                _close(c, ref, bound, torch.float32)
 
 
 @pytest.mark.gpu

@@ -24,6 +24,7 @@ struct MmParams {
   int epi;
   int out_dt, z_dt;
   int vec_z;
+  int fix;
 };
 
 // Tile shapes 64 RT x 64 CT (the "d" form with a deeper ring of stages, for
@@ -89,24 +90,31 @@ bool mm_plan(const MmCall& c, MmPlan* pl) {
   if (c.Z && !is_float(c.z_dt)) return false;
   if (c.sc_n != 1) return false;
   const int es = fp8 ? 1 : 2, al = 16 / es, bk = 128 / es;
-  // k-contiguous operands: 16-byte pieces along k, none across K's end;
-  // row-contiguous ones along the rows.  The copies' 32-bit offsets reach over
-  // one tile's rows or one step's k rows.
-  const auto mode = [&](const void* p, long long sb, long long sr, long long sk, bool* rc) {
-    if (!aligned16(p) || (c.batch > 1 && sb % al)) return false;
+  // operands contiguous along k or along the rows.  The copies' 32-bit offsets
+  // reach over one tile's rows or one step's k rows.  Pieces that no copy may
+  // take whole are filled by elements (gemm_pipe.h): the one across K's end
+  // of k-contiguous rows, and of row-contiguous operands that do not start on
+  // 16 bytes the one across the end of the last k row.
+  pl->fix = 0;
+  const auto mode = [&](const void* p, long long sb, long long sr, long long sk, int kbit,
+                        bool* rc) {
+    const bool al16 = aligned16(p) && (c.batch == 1 || sb % al == 0);
     const long long lim = 0x7f000000LL / es;
-    if (sk == 1 && sr % al == 0 && c.K % al == 0 && sr > 0 && sr < lim / 256 && c.K < lim / 2) {
+    if ((uintptr_t)p % es) return false;
+    if (sk == 1 && sr > 0 && sr < lim / 256 && c.K < lim / 2) {
       *rc = false;
+      if (c.K % al) pl->fix |= kbit;
       return true;
     }
-    if (sr == 1 && sk % al == 0 && sk > 0 && sk < lim / (bk + 1)) {
+    if (sr == 1 && sk >= al && sk < lim / (bk + 1)) {  // a piece reaches into one more row at most
       *rc = true;
+      if (!al16 || sk % al) pl->fix |= kbit << 2;
       return true;
     }
     return false;
   };
-  if (!mode(c.A, c.sa_b, c.sa_m, c.sa_k, &pl->arc) ||
-      !mode(c.B, c.sb_b, c.sb_n, c.sb_k, &pl->brc))
+  if (!mode(c.A, c.sa_b, c.sa_m, c.sa_k, 1, &pl->arc) ||
+      !mode(c.B, c.sb_b, c.sb_n, c.sb_k, 2, &pl->brc))
     return false;
   const int steps = (c.K + bk - 1) / bk;
   double best = 0;
@@ -143,6 +151,7 @@ int mm_launch(const MmCall& c, const MmPlan& pl, void* stream) {
   p.epi = c.Z ? 1 : 0;
   p.out_dt = c.out_dt; p.z_dt = c.z_dt;
   p.vec_z = c.Z && c.sz_n == 1;
+  p.fix = pl.fix;
   return launch(kernel_named(pl.name), dim3((unsigned)(pl.tiles_m * (long long)pl.tiles_n),
                                             (unsigned)c.batch),
                 dim3(256), 0, stream, p);

@@ -131,6 +131,7 @@ struct MmPlan {
   const char* tile;
   int tiles_m, tiles_n;
   bool arc, brc;  // operand row-contiguous (else k-contiguous)
+  int fix;        // pieces filled by elements (FIX_* of gemm_pipe.h)
 };
 // The kernel for a call (pointers only inspected for their alignment), or
 // false when these kernels do not take it; then its launch.

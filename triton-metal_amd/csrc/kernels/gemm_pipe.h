@@ -21,11 +21,18 @@ struct MmParams {
   int epi;           // 0: Z unused; else + Z (add-rows / -cols: sz_n / sz_m 0)
   int out_dt, z_dt;  // TM_DT_F32 / F16 / BF16
   int vec_z;         // Z's columns contiguous (sz_n 1)
+  int fix;           // pieces that no copy may take whole (FIX_*)
 };
 
 namespace mm {
 
 enum { F16 = 0, BF16 = 1, E4M3 = 2, E5M2 = 3 };
+
+// MmParams::fix: a k-contiguous operand whose K is no whole number of 16-byte
+// pieces; a row-contiguous one whose rows do not start on 16 bytes (a piece
+// across the end of its last k row could reach into another page).  Those
+// pieces are filled by element loads.
+enum { FIX_AK = 1, FIX_BK = 2, FIX_AR = 4, FIX_BR = 8 };
 
 typedef short s4v_t __attribute__((ext_vector_type(4)));
 typedef int i2v_t __attribute__((ext_vector_type(2)));
@@ -41,7 +48,8 @@ typedef __attribute__((address_space(3))) float lds_f_t;
 constexpr uint32_t kOob = 0x80000000u;
 
 // Global -> LDS copy through a buffer descriptor: lane l deposits 16 bytes at
-// lds + 16 l, zeros where voff is past the buffer.  Issued in asm for the
+// lds + 16 l (the source at any alignment of its elements), zeros where a dword
+// is past the buffer.  Issued in asm for the
 // reasons dma16 is (common.h); waited for with wait_vm.
 TM_DEV void buf16(u4_t rsrc, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff),
@@ -97,14 +105,41 @@ template <int KIND, bool RC, int R> struct Tile {
       return p * (16 / ES) < rows ? (uint32_t)kr * (uint32_t)ld * ES + 16u * p : kOob;
     }
   }
-  // whether copy i's piece starts before k = left of the step
+  // whether copy i's piece lies before k = left of the step
   static TM_DEV bool in_k(int wave, int lane, int i, int left) {
     const int blk = NCP * wave + i;
     if constexpr (!RC) {
       const int r = 8 * blk + (lane >> 3), p = (lane & 7) ^ ((r >> 1) & 7);
-      return p * (16 / ES) < left;
+      return (p + 1) * (16 / ES) <= left;
     } else {
       return (64 * blk + lane) / PPR < left;
+    }
+  }
+  // One piece of the stage at LDS `st` from n elements at src, zeros after
+  static TM_DEV void piece(uint32_t dst, const uint8_t* src, int n) {
+    u4_t v = {0u, 0u, 0u, 0u};
+    for (int e = 0; e < n; ++e) {
+      const uint32_t x = ES == 2 ? ((const uint16_t*)src)[e] : src[e];
+      const int at = e * ES;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        if ((at >> 2) == d) v[d] |= x << (8 * (at & 3));
+    }
+    *(lds_u4_t*)(dst) = v;
+  }
+  // The pieces of the last step that the copies left out: base = the tile's
+  // first row (column) at the step's k, kl = k left (1 .. BK), rows as voff
+  static TM_DEV void fill(uint32_t st, const uint8_t* base, int ld, int kl, int rows, int tid) {
+    constexpr int EP = 16 / ES;
+    if constexpr (!RC) {
+      const int pc = kl / EP;
+      for (int r = tid; r < ROWS; r += 256)
+        piece(st + 128 * r + 16 * (pc ^ ((r >> 1) & 7)),
+              base + ((size_t)r * ld + pc * EP) * ES, r < rows ? kl - pc * EP : 0);
+    } else if (rows % EP && tid == 0) {
+      const int pc = rows / EP, kr = kl - 1;
+      piece(st + RB * kr + 16 * (pc ^ sw_rc(kr)), base + ((size_t)kr * ld + pc * EP) * ES,
+            rows - pc * EP);
     }
   }
 };
@@ -254,6 +289,7 @@ __device__ __forceinline__ void mm_body(const MmParams& p) {
   // element (the bounds check drops whole dwords)
   constexpr int EP = 16 / ES;
   const int arp = (ar + EP - 1) / EP * EP, brp = (br + EP - 1) / EP * EP;
+  const int arl = (p.fix & FIX_AR) ? ar : arp, brl = (p.fix & FIX_BR) ? br : brp;  // last step
   const size_t astep = ARC ? (size_t)p.lda * BK * ES : 128u;
   const size_t bstep = BRC ? (size_t)p.ldb * BK * ES : 128u;
   uint32_t av[TA::NCP], bv[TB::NCP];
@@ -273,14 +309,14 @@ __device__ __forceinline__ void mm_body(const MmParams& p) {
     if constexpr (i < TA::NCP) {
       const uint32_t v = TA::in_k(wave, lane, i, left) ? av[i] : kOob;
       const u4_t r = buf_rsrc(abase + ks * astep,
-                              ARC ? ((uint32_t)((kl < BK ? kl : BK) - 1) * p.lda + arp) * ES
+                              ARC ? ((uint32_t)((kl < BK ? kl : BK) - 1) * p.lda + (ks + 1 < nk ? arp : arl)) * ES
                                   : ((uint32_t)(ar - 1) * p.lda + kl) * ES);
       buf16(r, v, la + s * STA + 1024 * i);
     } else {
       constexpr int j = i - TA::NCP;
       const uint32_t v = TB::in_k(wave, lane, j, left) ? bv[j] : kOob;
       const u4_t r = buf_rsrc(bbase + ks * bstep,
-                              BRC ? ((uint32_t)((kl < BK ? kl : BK) - 1) * p.ldb + brp) * ES
+                              BRC ? ((uint32_t)((kl < BK ? kl : BK) - 1) * p.ldb + (ks + 1 < nk ? brp : brl)) * ES
                                   : ((uint32_t)(br - 1) * p.ldb + kl) * ES);
       buf16(r, v, lb + s * STB + 1024 * j);
     }
@@ -327,6 +363,16 @@ __device__ __forceinline__ void mm_body(const MmParams& p) {
   static_for<0, NC1>([&](auto i) { copy(i, NS - 1, NS - 1); });
   wait_vm<(NS - 2) * NC + NC1>();
   asm volatile("s_barrier" ::: "memory");
+  // the last step's pieces that the copies left out, once the step has landed
+  auto fill = [&](int s) {
+    const int kl = K - (nk - 1) * BK;
+    if (p.fix & (ARC ? FIX_AR : FIX_AK))
+      TA::fill(lds0 + s * STA, abase + (nk - 1) * astep, p.lda, kl, ar, tid);
+    if (p.fix & (BRC ? FIX_BR : FIX_BK))
+      TB::fill(lds0 + LDSB + s * STB, bbase + (nk - 1) * bstep, p.ldb, kl, br, tid);
+    lds_barrier();
+  };
+  if (p.fix && nk == 1) fill(0);
   {
     std::integral_constant<int, 0> z;
     static_for<0, RT + CT>([&](auto y) { rd(z, y, 0); });
@@ -369,6 +415,7 @@ __device__ __forceinline__ void mm_body(const MmParams& p) {
       });
     });
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * NC) : "memory");
+    if (p.fix && kt + 2 == nk) fill(st + up);
 #pragma unroll
     for (int q = 0; q < decltype(rda)::NAD; ++q) rda.ad[q] += up * STA;
 #pragma unroll
