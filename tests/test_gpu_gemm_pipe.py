@@ -172,7 +172,7 @@ def test_selection():
     assert k(4096, 4096, 4096) == "mm_f16_kr_44"
     assert k(4096, 4096, 4096, trans_b=True, in_dtype=torch.bfloat16) == "mm_bf16_kk_44"
     assert k(16, 11008, 4096, trans_b=True, bias=True) == "mm_f16_kk_11"
-    assert k(2000, 11008, 4096, trans_b=True) == "mm_f16_kk_22"
+    assert k(2000, 11008, 4096, trans_b=True) == "mm_f16_kk_42"
     assert {k(M, 4096, 4096)[-2:] for M in (64, 512, 1024, 2048, 4096)} >= {"11", "44"}
     # odd N is fine for [N, K] weights, not for rows of [K, N]
     assert k(300, 1001, 1024, trans_b=True).startswith("mm_f16_kk_")

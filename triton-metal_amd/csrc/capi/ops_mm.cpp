@@ -35,12 +35,14 @@ struct MmParams {
 // full MFMA load allow); `res` tiles share a CU; fixed ns per round for the
 // pipeline's fill and the epilogue.  The larger tile moves fewer bytes into LDS
 // per MFMA, the smaller ones leave less of the last round idle and wait less
-// where there are few tiles: us for 44 / 42 / 22 / 22d / 21 / 11
-//   4096 x 4096 x 4096    105 / 122 / 125 / 137 / 159 / 200
-//   2000 x 11008 x 4096   195 / 184 / 175 / 199 / 210 / 266
-//   1000 x 4096 x 4096    101 /  58 /  49 /  40 /  44 /  52
+// where there are few tiles: us for 44 / 42 / 22 / 22d / 21 / 11, weights and
+// activations coming from HBM
+//   4096 x 4096 x 4096    117 / 137 / 144 / 159 / 179 / 234
+//   2000 x 11008 x 4096   231 / 222 / 241 / 264 / 292 / 360
+//   3000 x 2700 x 8000    184 / 207 / 217 / 199 / 214 / 232
+//   1000 x 4096 x 4096     89 /  54 /  51 /  42 /  47 /  59
 //   1136 x 1968 x 1024     28 /  17 /  14 /  11 /  12 /  13
-//     16 x 11008 x 4096    74 /  44 /  42 /  28 /  24 /  19
+//     64 x 8192 x 4096     76 /  48 /  47 /  33 /  30 /  22
 struct TileCost {
   const char* name;
   int rt, ct, res;
@@ -49,12 +51,12 @@ struct TileCost {
   double fixed;
 };
 const TileCost kTiles[] = {
-    {"44", 4, 4, 1, 1000, 1520, 2200, 3000, 13500},
-    {"42", 4, 2, 1, 600, 900, 1200, 1750, 5500},
-    {"22", 2, 2, 2, 450, 480, 900, 920, 4000},
-    {"22d", 2, 2, 1, 350, 550, 650, 950, 3300},
-    {"21", 2, 1, 2, 300, 295, 550, 560, 2500},
-    {"11", 1, 1, 2, 235, 187, 450, 360, 2000},
+    {"44", 4, 4, 1, 1000, 1560, 2200, 3000, 13500},
+    {"42", 4, 2, 1, 600, 950, 1200, 1750, 5500},
+    {"22", 2, 2, 2, 450, 590, 900, 920, 4000},
+    {"22d", 2, 2, 1, 350, 600, 650, 950, 3300},
+    {"21", 2, 1, 2, 300, 340, 550, 560, 2500},
+    {"11", 1, 1, 2, 235, 215, 450, 360, 2000},
 };
 
 double tile_cost(const TileCost& t, long long tiles, int steps, bool fp8) {

@@ -469,6 +469,10 @@ __device__ __forceinline__ void mm_body(const MmParams& p) {
           const long long zi = zb + (long long)m * p.sz_m + n * p.sz_n;
           if (p.vec_z) {
             add8(p.Z, zi, p.z_dt, &x[t], &y[t]);
+          } else if (p.sz_n == 0) {
+            const float z = load_as_f32_rt(p.Z, zi, p.z_dt);
+            x[t] += z;
+            y[t] += z;
           } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
