@@ -71,16 +71,21 @@ void plan_split(int batch, int q_heads, int kv_heads, int cap, int page_size, bo
 // number the one whose rounds of resident waves (160 KB of LDS per CU over the
 // ring of a wave) take least.  In positions of a wave's time: 100 for its
 // start, 75 for the combining launch and more past the 32 slices that it
-// merges at once.  Against the plan above (us, fp16, 16-position pages unless
-// said): 16 sequences of 2.5 to 8 k positions, 8 KV heads 146 -> 103 (8 slices
-// of 64 pages put 1024 waves on 768 places); 64 sequences of up to 1000, 64-
-// position pages 75 -> 60; 3 sequences of up to 2314, D = 96 23 -> 15 (9 slices left
-// most places empty).
+// merges at once.  With seq_lens (ragged) and at least 96 (sequence, KV head)
+// pairs a sequence is taken to fill two thirds of the capacity, and the slices
+// are an odd number: workgroups go to the 8 XCDs in turn, and of an even number
+// the late slices, empty for short sequences, all fall on the same XCDs.  (With
+// fewer pairs that makes too many slices to combine: 32 pairs 28 -> 39 us.)
+// Against the plan above (us, 16-position pages unless said): 16 sequences of
+// 2.5 to 8 k positions, 8 KV heads 146 -> 97 (8 slices of 64 pages; 6 slices
+// 103); 17 of 4 to 16 k, D = 64 93 -> 77; 64 of up to 1000, 64-position pages
+// 75 -> 60; 3 of up to 2314, D = 96 23 -> 15 (9 slices left most places empty).
 void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, int page_size,
-                 bool paged, int* nsplit, int* split_len) {
+                 bool paged, bool ragged, int* nsplit, int* split_len) {
   const int group = q_heads / kv_heads, hbn = (group + 15) / 16;
   const long long segs = (long long)batch * kv_heads * hbn;
   const long long slots = 256LL * (head_dim <= 64 ? 6 : 3);
+  ragged = ragged && segs >= 96;
   const int unit = slice_unit(page_size, paged);
   double best = 0;
   *nsplit = 0;
@@ -88,11 +93,14 @@ void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, in
     long long sl = (cap + n - 1) / n;
     sl = (sl + unit - 1) / unit * unit;
     if (n > 1 && sl < 64) break;
-    const double cost = (double)((segs * n + slots - 1) / slots) * (double)(sl + 100) +
+    const int slices = (int)((cap + sl - 1) / sl);
+    if (ragged && slices > 1 && slices % 2 == 0) continue;
+    const long long waves = ragged ? segs * (4 * n + 3) / 6 : segs * n;
+    const double cost = (double)((waves + slots - 1) / slots) * (double)(sl + 100) +
                         (n > 1 ? 75 + 2 * std::max(0, n - 32) : 0);
     if (*nsplit && cost >= best) continue;
     best = cost;
-    *nsplit = (int)((cap + sl - 1) / sl);
+    *nsplit = slices;
     *split_len = (int)sl;
   }
 }
@@ -120,7 +128,11 @@ extern "C" size_t tm_decode_attention_full_workspace_size(int batch, int q_heads
     return 0;
   int ns = 1, sl = 0;
   plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, page_size > 0 ? page_size : 1,
-              page_size > 0, &ns, &sl);
+              page_size > 0, false, &ns, &sl);
+  int nr = 1;
+  plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, page_size > 0 ? page_size : 1,
+              page_size > 0, true, &nr, &sl);
+  ns = std::max(ns, nr);
   return std::max(base, ns > 1 ? (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float)
                                : (size_t)0);
 }
@@ -196,7 +208,8 @@ static int decode_attention(const char* op, bool noalloc, const void* q, const v
         workspace_bytes >= tm_decode_attention_full_workspace_size(
                                batch, q_heads, kv_heads, head_dim, seq_len,
                                paged ? page_size : 0))
-      plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged, &ns, &sl);
+      plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged,
+                  seq_lens != nullptr, &ns, &sl);
     const size_t need = (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float);
     if (noalloc && ns > 1) {
       static DeviceGlobal scratch("tm_decode_scratch");
