@@ -77,3 +77,29 @@ def test_selection():
     # zero-points of int8, and groups other than 128, are not theirs
     assert not k(8, 11, 1280, 3456, zero_dtype=f16)["name"].startswith("wq_pipe")
     assert not k(4, 11, 1280, 3456, 64)["name"].startswith("wq_pipe")
+
+
+@pytest.mark.gpu
+def test_small_workspace_keeps_the_other_kernels():
+    """A workspace that the pipelined plan does not fit (too small for the slice
+    sums, then for the permuted X) is no error: one slice, then the kernels that
+    need none."""
+    import ctypes
+    from triton_metal_amd import _lib
+    L = _lib.lib()
+    M, N, K = 9, 272, 1152
+    x, w, s, z, deq, mag = _problem(4, M, N, K, torch.float16, "u", 3)
+    xd, wd, sd, zd = x.cuda(), w.cuda(), s.cuda(), z.cuda()
+    need = tm.wq_kernel_for(4, M, N, K, zero_dtype=torch.uint8, details=True)["workspace_bytes"]
+    ref = x.double() @ deq.t()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    for nbytes in (need, need - 1, M * K * 2 + 4096, 1024):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        rc = L.tm_wq_matmul_ws(4, p(xd), p(wd), None, p(y), p(sd), p(zd), M, N, K, 128,
+                               _lib.TM_DT_F16, _lib.TM_DT_F16, _lib.TM_DT_U8, p(ws), nbytes, None)
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        tol = 2.0 ** -11 * 1.01 * ref.abs() + 2.0 ** -24 * (K ** 0.5 * 4) * (x.double().abs()
+                                                                        @ mag.t()) + 1e-6
+        assert bool(((y.cpu().double() - ref).abs() <= tol).all()), nbytes

@@ -29,7 +29,8 @@ Kernel& kernel(const std::string& name) { return tmhip::kernel_named(name); }
 
 // ---- W-only kernel selection ------------------------------------------------
 // A pure function of the problem (sizes, dtypes, pointer alignment, the
-// device's CU count and LDS limit): the launch path and tm_wq_plan share it.
+// device's CU count and LDS limit, the workspace): the launch path and
+// tm_wq_plan share it.
 // Split-K plans (split_ok: the caller supplies a workspace) run the split-K
 // form of a kernel over `splits` k-slices, grid (grid, splits), writing fp32
 // [splits][M][N] into the workspace, then wq_splitk_reduce_<act>.
@@ -72,7 +73,7 @@ struct WqPipeParams {
 };
 
 void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, unsigned align,
-             int cus, size_t max_lds, bool split_ok, WqPlan* pl) {
+             int cus, size_t max_lds, bool split_ok, size_t ws_limit, WqPlan* pl) {
   pl->splits = 1;
   pl->kslice = K;
   pl->ws = 0;
@@ -94,6 +95,7 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
   // workspace for its copy of X), int8 without zero-points
   const bool pipe_ok = fast && K % 128 == 0 && (long long)K * 256 < (1LL << 31) &&
                        (qbits == 4 ? G == 128 && split_ok : zdt == TM_DT_NONE);
+  // (false: not within the caller's workspace)
   auto pipe = [&]() {
     const int rt = M <= 64 ? 1 : 2;
     const int tm = (M + 64 * rt - 1) / (64 * rt), tn = (N + 127) / 128, groups = K / 128;
@@ -105,11 +107,17 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
       per = (groups + want - 1) / want;
       S = (groups + per - 1) / per;
     }
+    if (wq_pipe_ws(qbits, M, N, K, S).total > ws_limit) {
+      S = 1;
+      per = groups;
+      if (wq_pipe_ws(qbits, M, N, K, S).total > ws_limit) return false;
+    }
     snprintf(pl->name, sizeof pl->name, "wq_pipe_q%d_%s_z%c_r%d", qbits, act, zc, rt);
     set((unsigned)(tm * tn), 256, 0, WQ_ARGS_PIPE);
     pl->splits = S;
     pl->kslice = per * 128;
     pl->ws = wq_pipe_ws(qbits, M, N, K, S).total;
+    return true;
   };
   // wide kernel (below): K in steps it can walk and aligned scales
   const bool w4k = qbits == 4 && (K % 512 == 0 || (K % 256 == 0 && zdt != TM_DT_U8));
@@ -123,8 +131,9 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
   // tiles 50 here 60, 392 109 here 88, 768 144 here 129; int8 M = 700: 240 tiles
   // 38 here 42, 288 63 here 56, 1032 167 here 153)
   const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (pipe_ok && M > 64 && t128 >= (!wide || (qbits == 4 && K > 4096) ? 160 : qbits == 4 ? 320 : 280))
-    return pipe();
+  if (pipe_ok && M > 64 && t128 >= (!wide || (qbits == 4 && K > 4096) ? 160 : qbits == 4 ? 320 : 280) &&
+      pipe())
+    return;
   // wide kernel: M > 64, 64 x 128 output blocks (int4: fp16 activations;
   // int8: fp16 or bf16).  With a workspace, split-K over S k-slices when its
   // tiles would fill less than half the CUs, or when int4 K exceeds the 4096
@@ -316,8 +325,9 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
   // -> 19, N = 3840 12 here 13; M = 228 K = 2816 N = 2816 26 -> 23, M = 28 K =
   // 1280 N = 1920 14 here 16: the permuting launch and the reduction cost 4)
   if (pipe_ok && (K % 256 != 0 || N % 64 != 0 ||
-                  (K <= 4096 && M > 1 && (long long)N * K >= (M > 64 ? 5000000 : 20000000))))
-    return pipe();
+                  (K <= 4096 && M > 1 && (long long)N * K >= (M > 64 ? 5000000 : 20000000))) &&
+      pipe())
+    return;
   // tiled kernel: 64 x 64 output tiles walking K in steps of 256.  With a
   // workspace and fewer tiles than CUs: split-K over slices of whole steps
   // (the last one shorter), about two workgroups per CU, at most 16 slices
@@ -375,7 +385,7 @@ int wq_matmul(int qbits, const void* X, const void* W, void* Y, const void* S, c
   const unsigned align = wq_align(X, W, S, Z);
   WqPlan pl;
   wq_plan(qbits, M, N, K, G, adt, sdt, zdt, align, cu_count(), (size_t)max_dynamic_lds(),
-          workspace != nullptr, &pl);
+          workspace != nullptr, workspace_bytes, &pl);
   if (pl.splits > 1 && workspace_bytes < pl.ws)
     return fail(TM_ERR_INVALID_ARG, "%s: workspace of %zu bytes, this call needs %zu", op,
                 workspace_bytes, pl.ws);
@@ -384,9 +394,6 @@ int wq_matmul(int qbits, const void* X, const void* W, void* Y, const void* S, c
   switch (pl.form) {
     case WQ_ARGS_PIPE: {
       const WqPipeWs w = wq_pipe_ws(qbits, M, N, K, pl.splits);
-      if (w.total > workspace_bytes)
-        return fail(TM_ERR_INVALID_ARG, "%s: workspace of %zu bytes, this call needs %zu", op,
-                    workspace_bytes, w.total);
       char* ws = (char*)workspace;
       WqPipeParams p;
       memset(&p, 0, sizeof p);
@@ -676,7 +683,7 @@ size_t tm_wq_workspace_bytes(int qbits, const void* input, const void* weight,
   WqPlan pl;
   wq_plan(qbits, M, N, K, qbits == 4 ? group_size : 1, act_dtype, scale_dtype, zero_dtype,
           wq_align(input, weight, scales, zeros), cu_count(), (size_t)max_dynamic_lds(), true,
-          &pl);
+          SIZE_MAX, &pl);
   return pl.ws;
 }
 
@@ -692,7 +699,7 @@ int tm_wq_plan(int qbits, int M, int N, int K, int group_size, int act_dtype, in
   clear_error();
   WqPlan pl;
   wq_plan(qbits, M, N, K, qbits == 4 ? group_size : 1, act_dtype, scale_dtype, zero_dtype,
-          align_flags, cu_count, max_lds, with_workspace != 0, &pl);
+          align_flags, cu_count, max_lds, with_workspace != 0, SIZE_MAX, &pl);
   if (name && name_len) snprintf(name, name_len, "%s", pl.name);
   if (grid) *grid = pl.grid;
   if (block) *block = pl.block;

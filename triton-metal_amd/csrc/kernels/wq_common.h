@@ -1,4 +1,4 @@
-// Helpers shared by the weight-only matmul kernels (wq_gemm.hip, wq_xreg.hip):
+// Helpers shared by the weight-only matmul kernels (wq_gemm.hip, wq_pipe.hip, ...):
 // scale / zero-point loads of a compile-time or runtime dtype, and the exact
 // 16-bit MFMA / dot operands built from int4 and int8 weights.
 #pragma once
