@@ -35,7 +35,7 @@ def _problem(qbits, M, N, K, act, zeros, seed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ACT)
 @pytest.mark.parametrize("qbits,zeros", [(4, None), (4, "s"), (4, "u"), (8, None)])
-@pytest.mark.parametrize("M,N,K", [(1, 144, 640), (2, 48, 128), (13, 272, 1152), (64, 128, 384),
+@pytest.mark.parametrize("M,N,K", [(1, 144, 640), (2, 48, 128), (40, 272, 1152), (64, 128, 384),
                                    (65, 400, 896), (129, 16, 2176), (200, 1040, 3200),
                                    (1300, 2064, 384)])
 def test_against_the_fp32_product(qbits, zeros, act, M, N, K):
@@ -68,15 +68,21 @@ def test_selection():
     assert k(4, 228, 2816, 7040, act_dtype=bf16)["name"] == "wq_pipe_q4_bf16_zn_r2"
     assert k(4, 1000, 4096, 11008, zero_dtype=u8)["name"] == "wq_pipe_q4_f16_zu_r2"
     assert k(4, 1000, 4096, 4096, zero_dtype=u8)["name"].startswith("wq_wide_")
-    assert k(8, 11, 1280, 3456)["name"] == "wq_pipe_q8_f16_zn_r1"
+    assert k(8, 40, 1280, 3456)["name"] == "wq_pipe_q8_f16_zn_r1"
     # without the workspace int4 stays where it was
     assert k(4, 228, 2816, 7040, with_workspace=False)["name"] == "wq_general"
     assert k(8, 700, 22016, 4096, with_workspace=False)["workspace_bytes"] == 0
-    d = k(4, 8, 1280, 3712)
-    assert d["splits"] > 1 and d["workspace_bytes"] >= d["splits"] * 8 * 1280 * 4 + 8 * 3712 * 2
+    d = k(4, 40, 1280, 3712)
+    assert d["splits"] > 1 and d["workspace_bytes"] >= d["splits"] * 40 * 1280 * 4 + 40 * 3712 * 2
+    # short K with few columns streams 16- / 32-column workgroups: K a multiple of
+    # 512 up to 64 rows, others up to 32
+    assert k(4, 64, 4096, 4096)["name"] == "wq_streamk_q4_f16_zn_t1_x16m_c4"
+    assert k(8, 16, 8192, 4096)["name"] == "wq_streamk_q8_f16_zn_t2_x16s_c8"
+    assert k(8, 32, 1280, 3456)["name"] == "wq_streamk_q8_f16_zn_t1_x16m_c8"
+    assert k(8, 16, 8208, 4096)["name"] == "wq_stream_q8_f16_zn_x16s"
     # zero-points of int8, and groups other than 128, are not theirs
-    assert not k(8, 11, 1280, 3456, zero_dtype=f16)["name"].startswith("wq_pipe")
-    assert not k(4, 11, 1280, 3456, 64)["name"].startswith("wq_pipe")
+    assert not k(8, 40, 1280, 3456, zero_dtype=f16)["name"].startswith("wq_pipe")
+    assert not k(4, 40, 1280, 3456, 64)["name"].startswith("wq_pipe")
 
 
 @pytest.mark.gpu
@@ -87,7 +93,7 @@ def test_small_workspace_keeps_the_other_kernels():
     import ctypes
     from triton_metal_amd import _lib
     L = _lib.lib()
-    M, N, K = 9, 272, 1152
+    M, N, K = 40, 272, 1152
     x, w, s, z, deq, mag = _problem(4, M, N, K, torch.float16, "u", 3)
     xd, wd, sd, zd = x.cuda(), w.cuda(), s.cuda(), z.cuda()
     need = tm.wq_kernel_for(4, M, N, K, zero_dtype=torch.uint8, details=True)["workspace_bytes"]

@@ -72,6 +72,23 @@ STREAMK = {
 for qb, shapes in STREAMK.items():
     for M, K, N in shapes:
         CASES += _each(qb, M, N, K)
+# the same kernel for short K (512 <= K <= 4096, at most 32 columns per CU: int4
+# 4, int8 8 chunks per wave): NT = 1 / 2, x8s / x16s / x16m, K with a partly
+# filled last round of chunks (1280 and 2176: 10 and 17 int4 chunks; 2880 and
+# 1600: 45 and 25 int8 ones), a last workgroup of one tile (N = 4112)
+STREAMK_SHORT = {
+    4: ((8, 4096, 1040), (2, 2176, 4096), (16, 1280, 48), (9, 3840, 2048), (64, 4096, 512),
+        (33, 512, 16), (7, 4096, 4112), (12, 2176, 8192), (40, 3072, 8176), (17, 512, 4112)),
+    8: ((8, 4096, 1040), (2, 2880, 4096), (16, 1600, 48), (9, 3840, 2048), (64, 4096, 512),
+        (33, 512, 16), (7, 4096, 4112), (12, 2880, 8192), (40, 3072, 8176), (17, 512, 4112)),
+}
+for qb, shapes in STREAMK_SHORT.items():
+    for M, K, N in shapes:
+        CASES += _each(qb, M, N, K)
+# the streaming kernels past 32 columns per CU
+for M, K in ((8, 1024), (12, 2048), (40, 512)):
+    CASES += _each(4, M, 8256, K)
+    CASES += _each(8, M, 8240, K)
 # its split-K forms (with a workspace): K past the single-launch limits in
 # two slices, one tile per workgroup; int4 x8 / x16 (K > 32768), x16m
 # (M > 16, K > 16384); int8 x8 / x16 / x16m (K > 16384)

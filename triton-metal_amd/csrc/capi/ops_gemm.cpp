@@ -200,10 +200,20 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
       return set(N / 32, 512, glds, WQ_ARGS_STD);
     }
   }
+  // K <= 4096 with at most 32 columns per CU (N <= 8192): the long-K kernel's
+  // 16- / 32-column workgroups below, in one round of the CUs; wider N would
+  // leave a second one partly filled and reads X more often (us, 48- / 64-column
+  // workgroups against 32-column ones, K = 4096: int8 M = 16 N = 8192 11.9 / 9.9,
+  // N = 10240 12.6 / 15.5; int4 M = 64 N = 8192 24.9 / 16.7, N = 10240 25.1 / 30.2)
+  // K not a multiple of 512: up to two passes of 16 rows, past that the pipelined
+  // kernel (us, its time against this one's: int8 K = 2816 N = 8192 M = 32 12.6 /
+  // 12.4, M = 64 15.0 / 19.0; int4 K = 3840 N = 4096 M = 32 14.6 / 8.8)
+  const bool narrow = M > 1 && M <= (K % 512 == 0 ? 64 : 32) && N / 16 <= 2 * cus &&
+                      K >= 512 && K <= 4096;
   // streaming kernel: 1 < M <= 64 (int4: 128), K-slices of 512 per wave (at
   // most 8); past 64 rows the int8 tiled kernel is the faster one
   if (fast && M > 1 && M <= (qbits == 4 ? 128 : 64) && K % 512 == 0 && K <= 4096 && sz4 &&
-      (qbits == 8 || G == 128)) {
+      (qbits == 8 || G == 128) && !narrow) {
     const int nwv = K / 512;
     const int nt = qbits == 4 ? 4 : 3;           // 16-column tiles per workgroup
     const int xr = M <= 8 ? 8 : 16;              // X rows staged per chunk
@@ -264,14 +274,14 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
       return set(N / 16, 512, glds, WQ_ARGS_STD);
     }
   }
-  // long-K streaming kernel: M <= 64, K > 4096 in chunks of 64 weight bytes
+  // long-K streaming kernel: M <= 64, K > 4096 (or few columns) in chunks of 64 weight bytes
   // per row (int4 128 k = one group, int8 64 k), NCH chunks per wave over at
   // most 8 waves (int4 K <= 32768, int8 K <= 16384); NT = 1 or 2 16-column
   // tiles per workgroup (one workgroup per CU for the N of a down projection;
-  // NT = 2 only where its LDS fits); M > 16 in passes of 16 rows (NT = 1;
+  // NT = 2 only where its LDS fits); M > 16 in passes of 16 rows (K > 4096: NT = 1;
   // int4 K <= 16384, as the first pass's weights stay in registers).  Past
   // those K, with a workspace: split-K over the fewest slices that fit.
-  if (fast && M <= 64 && K > 4096 && K % CK == 0 && sz4 && (qbits == 8 || G == 128)) {
+  if (fast && M <= 64 && (K > 4096 || narrow) && K % CK == 0 && sz4 && (qbits == 8 || G == 128)) {
     const bool multi = M > 16;
     const int kmax = qbits == 4 ? (multi ? 16384 : 32768) : 16384;
     int S = K <= kmax ? 1 : 0;
@@ -282,14 +292,16 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
     const int nchunk = Ks / CK;
     // split-K forms: int4 multi-pass 16 chunks per wave, the others 32
     const int nch = S > 1 ? (qbits == 4 && multi ? 16 : 32)
+                  : narrow ? (qbits == 4 ? 4 : 8)
                           : (nchunk <= 64 && qbits == 4 ? 8 : nchunk <= 128 ? 16 : 32);
     const int nwv = (nchunk + nch - 1) / nch;
     const int tiles = N / 16;
     const int xr = M <= 8 ? 8 : 16;
-    for (int nt = S == 1 && tiles > cus && !multi ? 2 : 1; S && nt >= 1; --nt) {
+    for (int nt = S == 1 && tiles > cus && (!multi || narrow) ? 2 : 1; S && nt >= 1; --nt) {
       const size_t slot = (size_t)nt * 1024 + (size_t)xr * 2 * CK;
       const size_t scb = qbits == 4 ? (size_t)512 * nt * (nch / 4) : 1024;
-      const size_t slds = (size_t)nwv * (2 * slot + scb + 8 * 64 * sizeof(float));
+      const int rs = !narrow ? 2 : qbits == 8 ? 4 : nt == 1 ? 3 : 2;  // ring slots per wave
+      const size_t slds = (size_t)nwv * (rs * slot + scb + 8 * 64 * sizeof(float));
       if (slds <= max_lds) {
         snprintf(pl->name, sizeof pl->name, "wq_streamk_q%d_%s_z%c_t%d_x%d%c_c%d%s", qbits, act,
                  zc, nt, xr, multi ? 'm' : 's', nch, S > 1 ? "_k" : "");
@@ -319,11 +331,10 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
     return set(N / 16, 256, lds, WQ_ARGS_G);
   }
   // K no multiple of 256 or N of 64 would run on wq_general (us, int4: M = 228
-  // K = 7040 N = 2816 1367 -> 30, M = 100 K = 9600 N = 4096 830 -> 31, M = 8 K =
-  // 3712 N = 1280 23 -> 14; int8 M = 11 K = 3456 31 -> 12).  K of at most 4096
+  // K = 7040 N = 2816 1367 -> 30, M = 100 K = 9600 N = 4096 830 -> 31).  K of at most 4096
   // that is a multiple of 256 only: larger weights (M = 3 K = 3840 N = 11520 28
-  // -> 19, N = 3840 12 here 13; M = 228 K = 2816 N = 2816 26 -> 23, M = 28 K =
-  // 1280 N = 1920 14 here 16: the permuting launch and the reduction cost 4)
+  // -> 19; M = 228 K = 2816 N = 2816 26 -> 23, smaller ones lose
+  // what the permuting launch and the reduction cost, 4)
   if (pipe_ok && (K % 256 != 0 || N % 64 != 0 ||
                   (K <= 4096 && M > 1 && (long long)N * K >= (M > 64 ? 5000000 : 20000000))) &&
       pipe())

@@ -1,11 +1,17 @@
 // W-only streaming kernel for long K: int4 (make_int4_matmul_kernel,
 // _msl_templates.py:2682-2745; weights [N, K/2] bytes, even k in the low
 // nibble) and int8 (make_int8_matmul_kernel, 2630-2679; weights [N, K]),
-// 2 <= M <= 64, K > 4096.
+// 2 <= M <= 64, K > 4096, and shorter K with at most 32 columns per CU.
 //
 // The down projections of a model (K = 11008, 14336, 28672, ...) have few
 // output columns, so the K <= 4096 streaming kernel's 48- / 64-column
-// workgroups would leave most CUs idle (N = 4096: 64 workgroups).  Here a
+// workgroups would leave most CUs idle (N = 4096: 64 workgroups); the output
+// and query / key / value projections of K <= 4096 are the same case.  What
+// bounds these is the latency of each wave's serial chunks, so short K takes few
+// chunks per wave (int4 4, int8 8: 8 waves at K = 4096) and a deeper ring (us at
+// K = N = 4096, fp16, weights from HBM, 48- / 64-column workgroups -> here: int8
+// M = 8 9.6 -> 6.2, M = 16 10.9 -> 6.9 (2.4 TB/s), M = 64 24.4 -> 14.0; int4 M = 16
+// 9.4 -> 5.7, M = 64 24.7 -> 12.9).  Here a
 // workgroup owns NT 16-column tiles (NT = 1 or 2: one workgroup per CU for
 // N = 4096 / 8192) and all of K: its nwv waves (at most 8) take the chunks
 // c = nwv i + w (i < NCH; int4 chunks are 128 k = one quantisation group,
@@ -14,7 +20,7 @@
 // LDS.  Chunks past the end (the last round when the chunk count is not a
 // multiple of nwv) re-read the last chunk and do not count.
 //
-// Per chunk a wave copies global -> LDS into a 2-slot ring of its own: the
+// Per chunk a wave copies global -> LDS into a ring of its own (2 to 4 slots): the
 // tiles' weights (16 rows x 64 B each, every 4 consecutive lanes on one
 // 64-byte segment) and the chunk's k of the XR activation rows; int4 scales /
 // zero-points (one dword per column and chunk) and int8 per-channel ones go to
@@ -60,7 +66,9 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
   constexpr int NJ = CK / 32;             // MFMA k-steps per chunk
   constexpr int XB = 2 * CK, XPR = XB / 16;
   constexpr int XI = XR * XPR / 64;       // X copies (1 KB each) per chunk
-  constexpr int RS = 2;                   // ring slots per wave
+  // ring slots per wave: short K (8 int8, 4 int4 chunks per wave) keeps what the
+  // LDS of a workgroup per CU takes in flight (the launch sizes its LDS alike)
+  constexpr int RS = QB == 4 ? (NCH == 4 && NT == 1 ? 3 : 2) : (NCH == 8 ? 4 : 2);
   constexpr int SLOT = NT * 1024 + XR * XB;
   constexpr int NQ = NCH / 4;             // int4 scale blocks (4 chunks x 16 columns)
   constexpr int SCB = QB == 4 ? 512 * NT * NQ : 1024;  // per-wave scales / zero-points
@@ -312,12 +320,13 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
 #define TM_STREAMK_A(QB, NT, XR, MS, MULTI, NCH)        \
   TM_STREAMK_Z(QB, false, f16, NT, XR, MS, MULTI, NCH)  \
   TM_STREAMK_Z(QB, true, bf16, NT, XR, MS, MULTI, NCH)
-// single pass (XR = 8 for M <= 8, 16 for M <= 16) and multi-pass (M <= 64,
-// NT = 1: the first pass's weight words stay in registers)
+// single pass (XR = 8 for M <= 8, 16 for M <= 16) and multi-pass (M <= 64; the
+// first pass's weight words stay in registers: NT = 1, short K also 2)
 #define TM_STREAMK_S(QB, NT, NCH)        \
   TM_STREAMK_A(QB, NT, 8, s, false, NCH) \
   TM_STREAMK_A(QB, NT, 16, s, false, NCH)
-#define TM_STREAMK_M(QB, NCH) TM_STREAMK_A(QB, 1, 16, m, true, NCH)
+#define TM_STREAMK_MN(QB, NT, NCH) TM_STREAMK_A(QB, NT, 16, m, true, NCH)
+#define TM_STREAMK_M(QB, NCH) TM_STREAMK_MN(QB, 1, NCH)
 // split-K forms (one 16-column tile per workgroup; the slices supply the
 // workgroups): single pass x8 / x16, multi-pass x16
 #define TM_STREAMK_SPLIT_Z(QB, BF, ACT, XR, MS, MULTI, NCH)                          \
