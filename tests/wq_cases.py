@@ -89,6 +89,9 @@ for qb, shapes in STREAMK_SHORT.items():
 for M, K in ((8, 1024), (12, 2048), (40, 512)):
     CASES += _each(4, M, 8256, K)
     CASES += _each(8, M, 8240, K)
+# two tiles per workgroup over several passes (8 int4 chunks per wave)
+for M, K, N in ((40, 5120, 4112), (17, 8192, 8176), (64, 6272, 5120)):
+    CASES += _each(4, M, N, K)
 # its split-K forms (with a workspace): K past the single-launch limits in
 # two slices, one tile per workgroup; int4 x8 / x16 (K > 32768), x16m
 # (M > 16, K > 16384); int8 x8 / x16 / x16m (K > 16384)

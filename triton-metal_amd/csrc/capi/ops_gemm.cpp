@@ -278,7 +278,8 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
   // per row (int4 128 k = one group, int8 64 k), NCH chunks per wave over at
   // most 8 waves (int4 K <= 32768, int8 K <= 16384); NT = 1 or 2 16-column
   // tiles per workgroup (one workgroup per CU for the N of a down projection;
-  // NT = 2 only where its LDS fits); M > 16 in passes of 16 rows (K > 4096: NT = 1;
+  // NT = 2 only where its LDS fits); M > 16 in passes of 16 rows (16 or
+  // 32 chunks per wave: NT = 1, two tiles' words do not fit the registers;
   // int4 K <= 16384, as the first pass's weights stay in registers).  Past
   // those K, with a workspace: split-K over the fewest slices that fit.
   if (fast && M <= 64 && (K > 4096 || narrow) && K % CK == 0 && sz4 && (qbits == 8 || G == 128)) {
@@ -297,7 +298,7 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
     const int nwv = (nchunk + nch - 1) / nch;
     const int tiles = N / 16;
     const int xr = M <= 8 ? 8 : 16;
-    for (int nt = S == 1 && tiles > cus && (!multi || narrow) ? 2 : 1; S && nt >= 1; --nt) {
+    for (int nt = S == 1 && tiles > cus && (!multi || nch <= 8) ? 2 : 1; S && nt >= 1; --nt) {
       const size_t slot = (size_t)nt * 1024 + (size_t)xr * 2 * CK;
       const size_t scb = qbits == 4 ? (size_t)512 * nt * (nch / 4) : 1024;
       const int rs = !narrow ? 2 : qbits == 8 ? 4 : nt == 1 ? 3 : 2;  // ring slots per wave

@@ -321,7 +321,10 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
   TM_STREAMK_Z(QB, false, f16, NT, XR, MS, MULTI, NCH)  \
   TM_STREAMK_Z(QB, true, bf16, NT, XR, MS, MULTI, NCH)
 // single pass (XR = 8 for M <= 8, 16 for M <= 16) and multi-pass (M <= 64; the
-// first pass's weight words stay in registers: NT = 1, short K also 2)
+// first pass's weight words stay in registers: NT = 2 up to 8 chunks per
+// wave; 16 int8 chunks of two tiles spill).  Two tiles halve the rounds past
+// 4096 columns: int4 K = 5120 N = 5120 M = 64 31.5 -> 24.8 us, K = 8192 N = 14336
+// M = 32 46.4 -> 34.4, 10240 columns (3 rounds of halves) the same
 #define TM_STREAMK_S(QB, NT, NCH)        \
   TM_STREAMK_A(QB, NT, 8, s, false, NCH) \
   TM_STREAMK_A(QB, NT, 16, s, false, NCH)

@@ -4,3 +4,4 @@
 TM_STREAMK_S(4, 1, 8)
 TM_STREAMK_S(4, 2, 8)
 TM_STREAMK_M(4, 8)
+TM_STREAMK_MN(4, 2, 8)
