@@ -61,6 +61,20 @@ def test_against_the_fp32_product(qbits, zeros, act, M, N, K):
     assert bool((err <= tol).all()), float((err / tol).max())
 
 
+@pytest.mark.gpu
+def test_more_rows_than_a_grid_dimension_holds():
+    """65536 rows and more (y and z of a grid end at 65535) on the pipelined int4
+    path, whose copy of X has one row of workgroups per row of X."""
+    M, N, K = 65600, 128, 256
+    assert tm.wq_kernel_for(4, M, N, K)[0] == "wq_pipe_q4_f16_zn_r2"
+    x, w, s, z, deq, _ = _problem(4, M, N, K, torch.float16, None, 9)
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    tm.int4_matmul(x.cuda(), w.cuda(), y, s.cuda(), None, M, N, K, 128)
+    ref = x.cuda().double() @ deq.t().contiguous().cuda()
+    err = (y.double() - ref).norm() / ref.norm()
+    assert err < 2 * 2.0 ** -11, float(err)  # one rounding to fp16
+
+
 def test_selection():
     """Sizes on both sides of the pipelined kernels' rules (no device is touched)."""
     k = lambda *a, **kw: tm.wq_kernel_for(*a, **kw, details=True)

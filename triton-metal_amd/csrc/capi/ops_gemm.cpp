@@ -418,7 +418,7 @@ int wq_matmul(int qbits, const void* X, const void* W, void* Y, const void* S, c
         p.SX = (const float*)(ws + w.sx);
         const int rc = launch(
             kernel(adt == TM_DT_BF16 ? "wq_pipe_prep_bf16" : "wq_pipe_prep_f16"),
-            dim3((unsigned)((K + 2047) / 2048), (unsigned)M), dim3(256), 0, stream, X, (void*)ws,
+            dim3((unsigned)M, (unsigned)((K + 2047) / 2048)), dim3(256), 0, stream, X, (void*)ws,
             (void*)(ws + w.sx), K, w.sxld);
         if (rc) return rc;
       }

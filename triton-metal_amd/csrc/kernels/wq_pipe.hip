@@ -41,10 +41,10 @@ struct WqPipeParams {
 };
 
 // X in operand order and the sums of its groups: a thread per 8 k, 16 threads
-// per group; grid (ceil(K / 2048), M).
+// per group; grid (M, ceil(K / 2048)): any number of rows (y holds 65535).
 template <bool BF16> TM_DEV void wq_pipe_prep_body(const uint16_t* X, uint16_t* XP, float* SX,
                                                    int K, int sxld) {
-  const int m = blockIdx.y, k = 2048 * blockIdx.x + 8 * threadIdx.x;
+  const int m = blockIdx.x, k = 2048 * blockIdx.y + 8 * threadIdx.x;
   if (k >= K) return;  // K % 128 == 0: whole groups of 16 lanes leave
   const u4_t x = ldg128(X + (size_t)m * K + k);
   float s = 0.0f;
