@@ -61,6 +61,55 @@ def test_against_the_fp32_product(qbits, zeros, act, M, N, K):
     assert bool((err <= tol).all()), float((err / tol).max())
 
 
+def _call(qbits, x, w, s, z, bias, general=False):
+    """y = x @ dequant(w)^T + bias; general: x two bytes off its alignment, which
+    leaves every kernel but wq_general (the sizes' former route)."""
+    M, K = x.shape
+    N = w.shape[0]
+    xd = x.cuda()
+    if general:
+        xd = torch.empty(M * K + 1, dtype=x.dtype, device="cuda")[1:].view(M, K).copy_(xd)
+        assert xd.data_ptr() % 4 == 2
+    y = torch.full((M, N), float("nan"), dtype=x.dtype, device="cuda")
+    wd, sd, zd, bd = (None if t is None else t.cuda() for t in (w, s, z, bias))
+    if qbits == 4:
+        tm.int4_linear(xd, wd, bd, y, sd, zd, M, N, K, 128)
+    else:
+        tm.int8_linear(xd, wd, bd, y, sd, zd, M, N, K)
+    return y.cpu().double()
+
+
+# (qbits, M, N, K): sizes that wq_general took before these kernels, K no
+# multiple of 256 or N of 64: the pipelined one and the short-K streaming ones
+NEW_ROUTES = [(4, 228, 272, 1152), (4, 100, 272, 7040), (4, 40, 144, 3200), (4, 3, 48, 640),
+              (4, 12, 4112, 1152), (4, 32, 272, 2176), (8, 5, 144, 1088), (8, 24, 272, 3264)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+@pytest.mark.parametrize("act", ACT)
+@pytest.mark.parametrize("zeros", [None, "s", "u"])
+@pytest.mark.parametrize("qbits,M,N,K", NEW_ROUTES)
+def test_no_further_from_64_bits_than_the_general_kernel(qbits, M, N, K, zeros, act, mean):
+    """The error against 64 bits (2-norm) is wq_general's, up to the few results
+    whose fp32 sum falls on the other side of a rounding (5e-4 of the error).
+    Zero-points near the middle of the weights, activations with a mean too."""
+    dt = ACT[act]
+    x, w, s, z, deq, _ = _problem(qbits, M, N, K, dt, None, M + N)
+    x = (x.float() + mean).to(dt)
+    if zeros:
+        z = 5 + 6 * torch.rand(s.shape, generator=torch.Generator().manual_seed(K))
+        z = z.round().to(torch.uint8) if zeros == "u" else z.to(dt)
+        rep = (1, 128) if qbits == 4 else (1, K)
+        wide = lambda t: t.double().reshape(N, -1).repeat_interleave(rep[1], 1)
+        deq = deq - wide(z) * wide(s)
+    name = tm.wq_kernel_for(qbits, M, N, K, act_dtype=dt, zero_dtype=None if z is None else z.dtype)
+    assert name[0] != "wq_general"
+    ref = x.double() @ deq.t()
+    err = [float((_call(qbits, x, w, s, z, None, general=g) - ref).norm()) for g in (False, True)]
+    assert err[0] <= err[1] * (1 + 5e-4), (name[0], err[0] / err[1])
+
+
 @pytest.mark.gpu
 def test_more_rows_than_a_grid_dimension_holds():
     """65536 rows and more (y and z of a grid end at 65535) on the pipelined int4

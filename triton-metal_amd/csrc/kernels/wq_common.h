@@ -67,6 +67,21 @@ TM_DEV u4_t w4_operand(uint32_t w, uint32_t mask, uint32_t magic) {
   r.w = ((w >> 12) & mask) | magic;
   return r;
 }
+// fp16 operands that leave the fp32 sums their bits, in the same order.
+// w4_operand64: 64 + q, the nibble at bits 4-7 of a half under 0x5400 (64, whose
+// ulp is 1/16), in as many instructions as 1024 + q.  w4_less: 1024 + q less c2 =
+// 1024 + z in every half is q - z for any uint8 z (whole numbers below 2048).
+// (The subnormal that a bare nibble is would need neither, but the MFMA keeps
+// fewer bits of it: its sums are no better than those of 1024 + q.)
+constexpr uint32_t kMask64 = 0x00F000F0u, kMagic64 = 0x54005400u;
+TM_DEV u4_t w4_operand64(uint32_t w, uint32_t mask, uint32_t magic, uint32_t s4, uint32_t s8) {
+  return u4_t{((w << s4) & mask) | magic, (w & mask) | magic, ((w >> s4) & mask) | magic,
+              ((w >> s8) & mask) | magic};
+}
+TM_DEV u4_t w4_less(u4_t o, h2_t c2) {
+  return u4_t{h2_bits(as_h2(o.x) - c2), h2_bits(as_h2(o.y) - c2), h2_bits(as_h2(o.z) - c2),
+              h2_bits(as_h2(o.w) - c2)};
+}
 template <bool BF16> constexpr uint32_t w4_magic() { return BF16 ? 0x43004300u : 0x64006400u; }
 template <bool BF16> constexpr float w4_offset() { return BF16 ? 128.0f : 1024.0f; }
 

@@ -12,11 +12,17 @@
 // A workgroup of 4 waves (2 x 2) owns 64 RT rows x 128 columns; K runs in
 // stages of 64 k through a three-stage LDS ring filled by bounds-checked
 // global -> LDS copies (rows past M or N deposit zeros).  The weights stay
-// packed in LDS and become exact 16-bit operands in registers (int4: OFF + q;
-// int8: q), so nothing is rounded before the fp32 sums: per group
-//   y += s (sum x (OFF + q) - (OFF + z) sum x)
-// with the group's sum x from wq_pipe_prep, which also writes X in the order
-// the int4 operands come out in (n0 n4 n1 n5 n2 n6 n3 n7 of each 8).
+// packed in LDS and become exact 16-bit operands in registers, so nothing is
+// rounded before the fp32 sums.  int8: q.  int4, per group
+//   y += s (sum x (q - c) - (z - c) sum x)
+// with c the centre of the operands and the group's sum x from wq_pipe_prep,
+// which also writes X in the order the int4 operands come out in (n0 n4 n1 n5 n2
+// n6 n3 n7 of each 8).  fp16: c = z without zero-points or with uint8 ones (one
+// packed subtraction per pair of operands and no second term), -64 with fp16 ones;
+// bf16: c = -128.  (c = -1024, the cheapest fp16 operand, left ten bits less to the
+// fp32 sums: relative error of the fp16 result at K = 7040 2.079e-4 against 2.076e-4
+// in exact sums, 2.084e-4 against 2.066e-4 for activations of mean 1.  bf16's sums
+// are 1.5e-6 off, a thousandth of the result's rounding.)
 // A lane holds one column per 32-column block (its scale is one register) and
 // 16 rows.  With a k slice per grid row the fp32 sums go to P[slice][M][N].
 // Two workgroups share a CU: the VALU work of one (per MFMA 4 operations of the
@@ -73,10 +79,13 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
   using namespace mm;
   constexpr int CT = 2, NS = 3, BM = 64 * RT, BN = 64 * CT;
   constexpr int WB = QB == 4 ? 32 : 64;            // weight bytes of a row per stage
-  constexpr int STX = BM * 128, STW = BN * WB, STS = QB == 4 ? 1024 : 0;
+  // int4 operands: q - z (fp16 with uint8 or no z); 64 + q (fp16), 128 + q (bf16),
+  // with a term left for the group's sums of x
+  constexpr bool LESS = QB == 4 && !BF16 && ZDT != TM_DT_F16, SUMX = QB == 4 && !LESS;
+  constexpr int STX = BM * 128, STW = BN * WB, STS = SUMX ? 1024 : 0;
   constexpr int ST = STX + STW + STS;
   constexpr int NCX = 2 * RT, NCW = STW / 4096;    // copies per wave
-  constexpr int NC = NCX + NCW + (QB == 4 ? 1 : 0);
+  constexpr int NC = NCX + NCW + (SUMX ? 1 : 0);
   constexpr int PW = WB / 16;                      // pieces of a weight row
   constexpr int LDW = 32 * CT + 4;
   constexpr int EPI = 4 * 32 * LDW * 4;
@@ -122,7 +131,7 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
 #pragma unroll
     for (int i = 0; i < NCW; ++i)
       buf16(rw, kt < nk ? wv[i] : kOob, base + STX + 1024 * (NCW * wave + i));
-    if constexpr (QB == 4) {
+    if constexpr (SUMX) {
       // the group's sums of x for this tile's rows (each wave copies the same
       // bytes to the same place)
       const int g = (k0 + 64 * ks) >> 7;
@@ -167,7 +176,8 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
   for (int j = 0; j < CT; ++j) col[j] = min(n0 + 32 * CT * wn + 32 * j + l32, p.N - 1);
   typename Raw<SDT>::T sraw[CT];
   typename Raw<ZDT>::T zraw[CT];
-  float sc[CT], zc[CT];
+  float sc[CT], zc[CT];  // scale and z - c
+  h2_t c2[CT];           // 1024 + z (LESS)
   auto load_sz = [&](int g) {
     if constexpr (QB == 4) {
       g = min(g, ng - 1);
@@ -183,7 +193,8 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
         sc[j] = raw_to_f32<SDT>(sraw[j]);
-        zc[j] = w4_offset<BF16>() + raw_to_f32<ZDT>(zraw[j]);
+        zc[j] = (LESS ? 1024.0f : BF16 ? 128.0f : 64.0f) + raw_to_f32<ZDT>(zraw[j]);
+        if constexpr (LESS) c2[j] = h2_t{(half_t)zc[j], (half_t)zc[j]};
       }
     }
   };
@@ -191,7 +202,8 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
   load_sz(k0 >> 7);
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) copies(s, s);
-  const uint32_t mask = vgpr_const(0x000F000Fu), magic = vgpr_const(w4_magic<BF16>());
+  const uint32_t mask = vgpr_const(SUMX && !BF16 ? kMask64 : 0x000F000Fu);
+  const uint32_t magic = vgpr_const(SUMX && !BF16 ? kMagic64 : w4_magic<BF16>());
   int st = 0, kt = 0;
   // one stage: wait for it, refill the slot read last, multiply
   auto stage = [&](bool first) {
@@ -212,8 +224,14 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int i = 0; i < RT; ++i) x[t][i] = *(lds_u4_t*)(xa[t] + off + 4096 * i);
+    if (LESS && first) {
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) acc[i][j] = f16_t{};
+    }
     f4_t sx[RT][4];
-    if (QB == 4 && first) {
+    if (SUMX && first) {
 #pragma unroll
       for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -230,7 +248,9 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
       u4_t o[CT];
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
-        if constexpr (QB == 4) o[j] = w4_operand(w[0][j][t], mask, magic);
+        if constexpr (LESS) o[j] = w4_less(w4_operand(w[0][j][t], mask, magic), c2[j]);
+        else if constexpr (QB == 4 && BF16) o[j] = w4_operand(w[0][j][t], mask, magic);
+        else if constexpr (QB == 4) o[j] = w4_operand64(w[0][j][t], mask, magic, 4, 8);
         else o[j] = w8_operand<BF16>(w[t >> 1][j][2 * (t & 1)], w[t >> 1][j][2 * (t & 1) + 1]);
       }
 #pragma unroll

@@ -30,7 +30,9 @@
 //   X piece p of row r at XB r + 16 (p ^ xsw(r))
 // Products on v_mfma_f32_16x16x32 (A = the activations, B = exact 16-bit
 // operands: int4 OFF + q, int8 q), the row sums of X on the same MFMA against
-// an all-ones B.  int4: per chunk y += s (sum x (OFF + q) - (OFF + z) sum x);
+// an all-ones B.  int4: per chunk y += s (sum x (OFF + q) - (OFF + z) sum x), OFF
+// 128 for bf16, 1024 for fp16 and, at K <= 4096, 64 for fp16 (some of these sizes
+// would run on wq_general, whose sums carry no offset; see wq_pipe.hip).
 // int8: y = s (sum x q - z sum x) at the end.  MULTI (M > 16): passes of 16
 // activation rows; the first pass keeps the weight words in registers, the
 // later ones stream only X.
@@ -75,6 +77,7 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
   constexpr int WB = RS * SLOT + SCB;
   constexpr int C0 = NT + XI, C1 = XI;    // copies per first- / later-pass chunk
   constexpr int NF = 4 * NT;              // partial sums per lane per pass
+  constexpr bool OFF64 = QB == 4 && !BF16 && NCH == 4;  // operands of 64 + q
   static_assert(NCH % 4 == 0 && NCH >= RS && XI >= 1 && (!MULTI || XR == 16), "streamk shape");
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -159,7 +162,8 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
 
   auto run_pass = [&](auto FIRSTC, int p) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(FIRSTC)::value;
-    const uint32_t vmask = vgpr_const(0x000F000Fu), vmagic = vgpr_const(w4_magic<BF16>());
+    const uint32_t vmask = vgpr_const(OFF64 ? kMask64 : 0x000F000Fu);
+    const uint32_t vmagic = vgpr_const(OFF64 ? kMagic64 : w4_magic<BF16>());
     const uint32_t s4 = vgpr_const(4u), s8 = vgpr_const(8u), s12 = vgpr_const(12u);
     const bool next = MULTI && p + 1 < npass;
     f4_t y[NT];
@@ -213,7 +217,8 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
           u4_t wop;
           if constexpr (QB == 4) {
             const uint32_t wj = j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w;
-            wop = w4_operand_v(wj, vmask, vmagic, s4, s8, s12);
+            wop = OFF64 ? w4_operand64(wj, vmask, vmagic, s4, s8)
+                        : w4_operand_v(wj, vmask, vmagic, s4, s8, s12);
           } else {
             // (opaque copies, so that the conversion stays in the pass loop)
             uint32_t w0 = j == 0 ? w.x : w.z, w1 = j == 0 ? w.y : w.w;
@@ -234,7 +239,7 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
           const size_t gi = (size_t)min(n0 + 16 * t + l16, N - 1) * srow + g0 + cc;
           float sc = raw_to_f32<SDT>((uint16_t)(*(const uint32_t*)sp2 >> (16 * (gi & 1))));
           sc = live ? sc : 0.0f;
-          float zb = w4_offset<BF16>();
+          float zb = OFF64 ? 64.0f : w4_offset<BF16>();
           if constexpr (ZDT == 3)
             zb += (float)((*(const uint32_t*)(sp2 + 256) >> (8 * (gi & 3))) & 0xFFu);
           else if constexpr (ZDT >= 0)
