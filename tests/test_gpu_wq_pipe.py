@@ -111,6 +111,39 @@ def test_no_further_from_64_bits_than_the_general_kernel(qbits, M, N, K, zeros, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("act", ACT)
+@pytest.mark.parametrize("zeros", [None, "s", "u"])
+@pytest.mark.parametrize("qbits,M,N,K", NEW_ROUTES + [(4, 700, 7168, 512), (8, 40, 272, 1152)])
+def test_infinite_activations(qbits, M, N, K, zeros, act):
+    """An infinite activation gives an infinity of the weight's sign (NaN for a weight
+    of exactly its zero-point), two of opposite signs NaN where they meet, and
+    activations whose multiples overflow the sums stay finite: all as wq_general.
+    Rows without one are untouched."""
+    dt = ACT[act]
+    x, w, s, z, deq, mag = _problem(qbits, M, N, K, dt, zeros, M + K)
+    inf = float("inf")
+    clean = _call(qbits, x, w, s, z, None)
+    x[0, 5] = inf
+    x[1, K - 1] = -inf
+    x[2, 7], x[2, K - 70] = inf, inf
+    x[M - 1, 3] = float("nan")
+    if M > 4:
+        x[3, 100], x[3, 101] = -inf, torch.finfo(dt).max
+        x[M - 2, K // 2] = torch.finfo(dt).max / 64
+    got, want = _call(qbits, x, w, s, z, None), _call(qbits, x, w, s, z, None, general=True)
+    assert bool((got.isnan() == want.isnan()).all())
+    assert bool((got.isinf() == want.isinf()).all())
+    i = want.isinf()
+    assert i.any() and torch.equal(got[i], want[i])
+    f = want.isfinite()
+    u = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    # a rounding apart, and the sums' own error (partial sums of at most x (OFF + q + z) s)
+    tol = 2 * u * want[f].abs() + 2.0 ** -24 * (x.double().abs().nan_to_num(0, 0) @ mag.t())[f]
+    assert bool(((got[f] - want[f]).abs() <= tol + 1e-6).all())
+    assert torch.equal(got[4:M - 2], clean[4:M - 2])
+
+
+@pytest.mark.gpu
 def test_more_rows_than_a_grid_dimension_holds():
     """65536 rows and more (y and z of a grid end at 65535) on the pipelined int4
     path, whose copy of X has one row of workgroups per row of X."""

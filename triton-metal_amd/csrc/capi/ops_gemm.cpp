@@ -61,6 +61,7 @@ WqPipeWs wq_pipe_ws(int qbits, int M, int N, int K, int splits) {
 }
 struct WqPipeParams {
   const void* X;
+  const void* X0;
   const void* W;
   const void* S;
   const void* Z;
@@ -409,7 +410,7 @@ int wq_matmul(int qbits, const void* X, const void* W, void* Y, const void* S, c
       char* ws = (char*)workspace;
       WqPipeParams p;
       memset(&p, 0, sizeof p);
-      p.X = X; p.W = W; p.S = S; p.Z = Z; p.Y = Y; p.bias = bias;
+      p.X = p.X0 = X; p.W = W; p.S = S; p.Z = Z; p.Y = Y; p.bias = bias;
       p.M = M; p.N = N; p.K = K; p.kslice = pl.kslice; p.sxld = w.sxld;
       p.tiles_n = (N + 127) / 128;
       p.tiles_m = (int)pl.grid / p.tiles_n;

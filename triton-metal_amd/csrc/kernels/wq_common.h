@@ -196,4 +196,38 @@ TM_DEV float xsum8(u4_t v, bool bf16) {
   }
   return a;
 }
+
+// sum over k0 <= k < k1 of x[k] (q[k] - z) s in wq_general's own form, by the whole
+// wave (8 k a lane; k1 - k0 a multiple of 8): one output that came out infinite or
+// NaN where its sums run over x OFF, x q and z x apart, which meet as inf - inf for
+// an infinite x (or one whose multiple overflows) while the products here keep
+// their signs.  x, w: the output's rows; si: the row's first scale (int4: a group
+// of 128 k each).
+template <int QB, bool BF16, int ZDT>
+TM_DEV float wq_direct(const uint16_t* x, const uint8_t* w, const void* S, const void* Z,
+                       size_t si, int k0, int k1, int lane) {
+  constexpr int SDT = BF16 ? TM_DT_BF16 : TM_DT_F16;
+  float acc = 0.0f;
+  for (int kb = k0; kb < k1; kb += 512) {
+    const int k = kb + 8 * lane;
+    if (k < k1) {
+      const u4_t xv = ldg128(x + k);
+      const size_t g = QB == 4 ? si + (k >> 7) : si;
+      const float sc = ld_typed<SDT>(S, g), zp = ld_typed<ZDT>(Z, g);
+      uint32_t wd[2] = {*(const uint32_t*)(w + (QB == 4 ? k / 2 : k)), 0};
+      if constexpr (QB == 8) wd[1] = *(const uint32_t*)(w + k + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint16_t b = (uint16_t)(xv[e >> 1] >> (16 * (e & 1)));
+        const float xf = BF16 ? bf16_bits_to_f32(b) : f16_bits_to_f32(b);
+        const float q = QB == 4 ? (float)((wd[0] >> (4 * e)) & 15u)
+                                : (float)(int8_t)(wd[e >> 2] >> (8 * (e & 3)));
+        acc += xf * ((q - zp) * sc);
+      }
+    }
+    if (__ballot(acc != acc)) break;  // NaN stays NaN
+  }
+  return wave_sum(acc);
+}
+TM_DEV bool not_finite(float v) { return !(__builtin_fabsf(v) < INFINITY); }
 }  // namespace

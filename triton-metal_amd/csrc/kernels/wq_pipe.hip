@@ -35,6 +35,7 @@
 
 struct WqPipeParams {
   const void* X;       // [M, K], int4: as wq_pipe_prep writes it
+  const uint16_t* X0;  // [M, K] as the caller has it
   const uint8_t* W;
   const void* S;
   const void* Z;
@@ -302,7 +303,29 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
       const int r = t * (64 / LPR) + lane / LPR, m = mw + 32 * i + r;
       f4_t a = *(lds_f4_t*)(eb + 4u * (r * LDW + c));
       f4_t b = *(lds_f4_t*)(eb + 4u * (r * LDW + c + 4));
-      if (m >= p.M || n >= p.N) continue;
+      const bool in = m < p.M && n < p.N;
+      if constexpr (!LESS) {
+        // infinite and NaN outputs again as wq_general sums them (wq_direct)
+        bool bad = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad |= not_finite(a[e]) || not_finite(b[e]);
+        for (uint64_t todo = __ballot(in && bad); todo; todo &= todo - 1) {
+          const int l = __builtin_ctzll(todo), ml = __builtin_amdgcn_readlane(m, l),
+                    nl = __builtin_amdgcn_readlane(n, l);
+          for (int e = 0; e < 8; ++e) {
+            const float v = e < 4 ? a[e & 3] : b[e & 3];
+            if (!((__ballot(not_finite(v)) >> l) & 1)) continue;
+            const float d = wq_direct<QB, BF16, ZDT>(
+                p.X0 + (size_t)ml * K, p.W + (size_t)(nl + e) * wrow, p.S, p.Z,
+                (size_t)(nl + e) * (QB == 4 ? ng : 1), k0, k1, lane);
+            if (lane == l) {
+              if (e < 4) a[e & 3] = d;
+              else b[e & 3] = d;
+            }
+          }
+        }
+      }
+      if (!in) continue;
       const size_t o = (size_t)m * p.N + n;
       if (P) {
         *(f4_t*)(P + o) = a;

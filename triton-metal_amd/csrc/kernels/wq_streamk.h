@@ -78,6 +78,8 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
   constexpr int C0 = NT + XI, C1 = XI;    // copies per first- / later-pass chunk
   constexpr int NF = 4 * NT;              // partial sums per lane per pass
   constexpr bool OFF64 = QB == 4 && !BF16 && NCH == 4;  // operands of 64 + q
+  // outputs that are not finite again, as wq_general sums them
+  constexpr bool REDO = NCH == (QB == 4 ? 4 : 8);
   static_assert(NCH % 4 == 0 && NCH >= RS && XI >= 1 && (!MULTI || XR == 16), "streamk shape");
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -288,6 +290,16 @@ __device__ __forceinline__ void wq_streamk_body(const uint16_t* X, const uint8_t
         for (int w2 = 0; w2 < nwv; ++w2) v += red[(w2 * 8 + f) * 64 + lane];
         const int F = 8 * r + f, t = F >> 2, e = F & 3;
         const int row = 16 * p + 4 * q + e, col = n0 + 16 * t + l16;
+        if constexpr (REDO) {
+          for (uint64_t todo = __ballot(row < M && col < N && not_finite(v)); todo;
+               todo &= todo - 1) {
+            const int l = __builtin_ctzll(todo), nl = __builtin_amdgcn_readlane(col, l);
+            const float d = wq_direct<QB, BF16, ZDT>(
+                X + (size_t)__builtin_amdgcn_readlane(row, l) * K, W + (size_t)nl * rowbytes, S, Z,
+                (size_t)nl * (QB == 4 ? srow : 1), 0, K, lane);
+            if (lane == l) v = d;
+          }
+        }
         if (row < M && col < N) {
           if constexpr (SPLIT) P[((size_t)blockIdx.y * M + row) * N + col] = v;
           else store_out(Y, (size_t)row * N + col, v + bias_at(bias, col, BF16), BF16);
