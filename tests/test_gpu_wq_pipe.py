@@ -9,6 +9,10 @@ ACT = {"f16": torch.float16, "bf16": torch.bfloat16}
 
 
 def _problem(qbits, M, N, K, act, zeros, seed):
+    """x, weights, scales, zero-points, the dequantised weights, and the largest
+    terms the kernels sum in fp32: (OFF + q + z) s, OFF the operands' offset (a
+    single fp16 row: the GEMV kernels, 1024)."""
+    off = 0 if qbits == 8 else 128 if act == torch.bfloat16 else 64 if M > 1 else 1024
     g = torch.Generator().manual_seed(seed)
     x = torch.randn(M, K, generator=g).to(act)
     cols = K // 128 if qbits == 4 else 1
@@ -26,10 +30,18 @@ def _problem(qbits, M, N, K, act, zeros, seed):
         z = (torch.rand(N, cols, generator=g) * 15).to(act)
     rep = K // cols
     deq = s.double().repeat_interleave(rep, 1)
-    mag = (q.abs() + (0 if z is None else z.double().repeat_interleave(rep, 1)) +
-           (1024 if qbits == 4 else 0)) * deq
+    mag = (q.abs() + (0 if z is None else z.double().repeat_interleave(rep, 1)) + off) * deq
     deq = deq * (q - (0 if z is None else z.double().repeat_interleave(rep, 1)))
     return x, w, s if qbits == 4 else s.reshape(N), z, deq, mag
+
+
+def _sum_bound(x, deq, mag):
+    """How far the fp32 sums may be off: each addition rounds a partial sum whose
+    size is that of the terms' 2-norm, in groups of 128 k (|x| mag) and then over the
+    groups (|x| deq); 16 and 4 for the largest of many outputs."""
+    x2 = x.double() ** 2
+    return 2.0 ** -24 * (16 * (x2 @ (mag ** 2).t()).sqrt()
+                         + 4 * (x.shape[1] / 128) ** 0.5 * (x2 @ (deq ** 2).t()).sqrt())
 
 
 @pytest.mark.gpu
@@ -54,11 +66,53 @@ def test_against_the_fp32_product(qbits, zeros, act, M, N, K):
     else:
         tm.int8_linear(xd, wd, bd, y, sd, zd, M, N, K)
     ref = x.double() @ deq.t() + bias.double()
-    # one rounding of the result, and fp32 sums of OFF + q and z sum x
+    # one rounding of the result on top of the sums'
     u = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
-    tol = 1.01 * u * ref.abs() + 2.0 ** -24 * (K ** 0.5 * 4) * (x.double().abs() @ mag.t()) + 1e-6
+    tol = 1.01 * u * ref.abs() + _sum_bound(x, deq, mag) + 1e-6
     err = (y.cpu().double() - ref).abs()
     assert bool((err <= tol).all()), float((err / tol).max())
+    # the sums themselves: equal rows with a bias that cancels them up to its own
+    # rounding leave a result small enough for the output type to show the error
+    x = x[:1].expand(M, K).contiguous()
+    ref = x[:1].double() @ deq.t()
+    bias = (-ref[0]).to(dt)
+    rest = ref + bias.double()
+    err = (_call(qbits, x, w, s, z, bias) - rest).abs()
+    tol = 1.01 * u * rest.abs() + _sum_bound(x[:1], deq, mag) + 1e-7
+    assert bool((err <= tol).all()), float((err / tol).max())
+
+
+@pytest.mark.parametrize("act", ACT)
+@pytest.mark.parametrize("zeros", [None, "s", "u"])
+@pytest.mark.parametrize("K", [128, 640, 3200])
+def test_the_bound_on_the_sums_sees_lost_bits(K, zeros, act):
+    """The bound of the test above holds for fp32 sums of the kernels' form and fails
+    for sums that lose bits: rounded to bf16 after each group (two groups and more),
+    or a scale that is 2^-12 off."""
+    dt = ACT[act]
+    M, N = 4, 64
+    x, w, s, z, deq, mag = _problem(4, M, N, K, dt, zeros, K)
+    off = 128.0 if act == "bf16" else 64.0
+    q = torch.stack((w & 15, w >> 4), -1).reshape(N, K).float()
+    zf = torch.zeros(N, K // 128) if z is None else z.float()
+    ref = x.double() @ deq.t()
+
+    def sums(keep, scale):
+        y = torch.zeros(M, N)
+        for g in range(K // 128):
+            xg, k = x[:, 128 * g:128 * g + 128].float(), slice(128 * g, 128 * g + 128)
+            acc = -(zf[:, g] + off) * xg.sum(1, keepdim=True)
+            for e in range(0, 128, 16):
+                acc = acc + xg[:, e:e + 16] @ (off + q[:, k][:, e:e + 16]).t()
+            y = keep(y + s[:, g].float() * scale * acc)
+        return (y.double() - ref).abs()
+
+    same = lambda t: t
+    bound = _sum_bound(x, deq, mag)
+    assert bool((sums(same, 1.0) <= bound).all())
+    assert not bool((sums(same, 1 + 2.0 ** -12) <= bound).all())
+    if K > 128:
+        assert not bool((sums(lambda t: t.bfloat16().float(), 1.0) <= bound).all())
 
 
 def _call(qbits, x, w, s, z, bias, general=False):
@@ -138,7 +192,7 @@ def test_infinite_activations(qbits, M, N, K, zeros, act):
     f = want.isfinite()
     u = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
     # a rounding apart, and the sums' own error (partial sums of at most x (OFF + q + z) s)
-    tol = 2 * u * want[f].abs() + 2.0 ** -24 * (x.double().abs().nan_to_num(0, 0) @ mag.t())[f]
+    tol = 2 * u * want[f].abs() + 2 * _sum_bound(x.nan_to_num(0, 0, 0), deq, mag)[f]
     assert bool(((got[f] - want[f]).abs() <= tol + 1e-6).all())
     assert torch.equal(got[4:M - 2], clean[4:M - 2])
 
@@ -202,6 +256,5 @@ def test_small_workspace_keeps_the_other_kernels():
                                _lib.TM_DT_F16, _lib.TM_DT_F16, _lib.TM_DT_U8, p(ws), nbytes, None)
         assert rc == 0, _lib.last_error()
         torch.cuda.synchronize()
-        tol = 2.0 ** -11 * 1.01 * ref.abs() + 2.0 ** -24 * (K ** 0.5 * 4) * (x.double().abs()
-                                                                        @ mag.t()) + 1e-6
+        tol = 2.0 ** -11 * 1.01 * ref.abs() + _sum_bound(x, deq, mag) + 1e-6
         assert bool(((y.cpu().double() - ref).abs() <= tol).all()), nbytes
