@@ -71,21 +71,21 @@ void plan_split(int batch, int q_heads, int kv_heads, int cap, int page_size, bo
 // number the one whose rounds of resident waves (160 KB of LDS per CU over the
 // ring of a wave) take least.  In positions of a wave's time: 100 for its
 // start, 75 for the combining launch and more past the 32 slices that it
-// merges at once.  With seq_lens (ragged) and at least 96 (sequence, KV head)
-// pairs a sequence is taken to fill two thirds of the capacity, and the slices
-// are an odd number: workgroups go to the 8 XCDs in turn, and of an even number
-// the late slices, empty for short sequences, all fall on the same XCDs.  (With
-// fewer pairs that makes too many slices to combine: 32 pairs 28 -> 39 us.)
-// Against the plan above (us, 16-position pages unless said): 16 sequences of
-// 2.5 to 8 k positions, 8 KV heads 146 -> 97 (8 slices of 64 pages; 6 slices
-// 103); 17 of 4 to 16 k, D = 64 93 -> 77; 64 of up to 1000, 64-position pages
-// 75 -> 60; 3 of up to 2314, D = 96 23 -> 15 (9 slices left most places empty).
+// merges at once.  Every sequence counts as full, also with seq_lens: the host
+// does not know the lengths, and a count made for shorter ones starts a second
+// round when they are not.  us for lengths all full / from a quarter of the
+// capacity to all of it / all a quarter, and the slices: 16 sequences of 8 KV heads,
+// 8192 in 16-position pages, the plan above 150 / 146 / 143 (8), made for two
+// thirds 165 / 95 / 92 (7), here 108 / 103 / 95 (6); 32 of 8, 4096 152 / 146 / 144 (4),
+// 137 / 97 / 57 (11), 112 / 103 / 73 (3); 17 of 8, 16384, D = 64 120 / 110 / 107 (16), 127
+// / 78 / 65, 98 / 86 / 80 (11); 45 of 4, 4494 in 64-position pages 132 / 78 / 75 (5),
+// 134 / 80 / 76 (5), 95 / 88 / 87 (4): an odd count spreads the empty slices better
+// over the XCDs, which take workgroups in turn.
 void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, int page_size,
-                 bool paged, bool ragged, int* nsplit, int* split_len) {
+                 bool paged, int* nsplit, int* split_len) {
   const int group = q_heads / kv_heads, hbn = (group + 15) / 16;
   const long long segs = (long long)batch * kv_heads * hbn;
   const long long slots = 256LL * (head_dim <= 64 ? 6 : 3);
-  ragged = ragged && segs >= 96;
   const int unit = slice_unit(page_size, paged);
   double best = 0;
   *nsplit = 0;
@@ -94,9 +94,7 @@ void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, in
     sl = (sl + unit - 1) / unit * unit;
     if (n > 1 && sl < 64) break;
     const int slices = (int)((cap + sl - 1) / sl);
-    if (ragged && slices > 1 && slices % 2 == 0) continue;
-    const long long waves = ragged ? segs * (4 * n + 3) / 6 : segs * n;
-    const double cost = (double)((waves + slots - 1) / slots) * (double)(sl + 100) +
+    const double cost = (double)((segs * n + slots - 1) / slots) * (double)(sl + 100) +
                         (n > 1 ? 75 + 2 * std::max(0, n - 32) : 0);
     if (*nsplit && cost >= best) continue;
     best = cost;
@@ -128,11 +126,7 @@ extern "C" size_t tm_decode_attention_full_workspace_size(int batch, int q_heads
     return 0;
   int ns = 1, sl = 0;
   plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, page_size > 0 ? page_size : 1,
-              page_size > 0, false, &ns, &sl);
-  int nr = 1;
-  plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, page_size > 0 ? page_size : 1,
-              page_size > 0, true, &nr, &sl);
-  ns = std::max(ns, nr);
+              page_size > 0, &ns, &sl);
   return std::max(base, ns > 1 ? (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float)
                                : (size_t)0);
 }
@@ -208,8 +202,7 @@ static int decode_attention(const char* op, bool noalloc, const void* q, const v
         workspace_bytes >= tm_decode_attention_full_workspace_size(
                                batch, q_heads, kv_heads, head_dim, seq_len,
                                paged ? page_size : 0))
-      plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged,
-                  seq_lens != nullptr, &ns, &sl);
+      plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged, &ns, &sl);
     const size_t need = (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float);
     if (noalloc && ns > 1) {
       static DeviceGlobal scratch("tm_decode_scratch");
