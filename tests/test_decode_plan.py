@@ -25,3 +25,11 @@ def test_full_sequences_take_one_round(B, Hkv, rep, D, S, page, want):
     every sequence is full where one round takes them all."""
     n = slices(B, Hkv, rep, D, S, page)
     assert n == want and rounds(B, Hkv, rep, D, n) == 1
+
+
+@pytest.mark.parametrize("Hkv,rep,S,page,most", [
+    (1, 8, 8192, 16, 32), (8, 4, 8192, 16, 32), (1, 8, 4096, 16, 32), (8, 4, 32768, 0, 96)])
+def test_few_sequences_do_not_outgrow_the_combining_kernel(Hkv, rep, S, page, most):
+    """More than the 32 slices that are merged at once only where the slices save more
+    than merging them one by one takes (64 of 8192 positions: 26.7 us, 32: 23.4)."""
+    assert most // 2 < slices(1, Hkv, rep, 128, S, page) <= most

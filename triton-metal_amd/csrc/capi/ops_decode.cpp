@@ -69,9 +69,11 @@ void plan_split(int batch, int q_heads, int kv_heads, int cap, int page_size, bo
 // Slices for the 16-bit kernels when the workspace has room for them
 // (tm_decode_attention_full_workspace_size): of any number of pages, their
 // number the one whose rounds of resident waves (160 KB of LDS per CU over the
-// ring of a wave) take least.  In positions of a wave's time: 100 for its
-// start, 75 for the combining launch and more past the 32 slices that it
-// merges at once.  Every sequence counts as full, also with seq_lens: the host
+// ring of a wave) take least.  In positions of a wave's time (about 60 ns paged, 45
+// contiguous): 100 for its start, 75 for the combining launch, and where that has
+// more slices than the 32 it merges at once 0.2 us for each of them (us, one
+// sequence of 8192 positions, 1 KV head: 32 slices 23.4, 40 29.4, 64 26.7; 8 heads 24.4,
+// 31.4, 29.6; of 32768, 8 heads: 32 slices 74, 64 60, 96 58).  Every sequence counts as full, also with seq_lens: the host
 // does not know the lengths, and a count made for shorter ones starts a second
 // round when they are not.  us for lengths all full / from a quarter of the
 // capacity to all of it / all a quarter, and the slices: 16 sequences of 8 KV heads,
@@ -95,7 +97,7 @@ void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, in
     if (n > 1 && sl < 64) break;
     const int slices = (int)((cap + sl - 1) / sl);
     const double cost = (double)((segs * n + slots - 1) / slots) * (double)(sl + 100) +
-                        (n > 1 ? 75 + 2 * std::max(0, n - 32) : 0);
+                        (n > 1 ? 75 : 0) + (n > 32 ? (paged ? 3.5 : 4.5) * n : 0);
     if (*nsplit && cost >= best) continue;
     best = cost;
     *nsplit = slices;
