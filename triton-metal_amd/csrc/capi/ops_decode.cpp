@@ -88,20 +88,38 @@ void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, in
   const int group = q_heads / kv_heads, hbn = (group + 15) / 16;
   const long long segs = (long long)batch * kv_heads * hbn;
   const long long slots = 256LL * (head_dim <= 64 ? 6 : 3);
-  const int unit = slice_unit(page_size, paged);
+  const unsigned unit = (unsigned)slice_unit(page_size, paged), ucap = (unsigned)cap;
   double best = 0;
   *nsplit = 0;
-  for (int n = 1; n <= 256; ++n) {
-    long long sl = (cap + n - 1) / n;
-    sl = (sl + unit - 1) / unit * unit;
-    if (n > 1 && sl < 64) break;
-    const int slices = (int)((cap + sl - 1) / sl);
-    const double cost = (double)((segs * n + slots - 1) / slots) * (double)(sl + 100) +
-                        (n > 1 ? 75 : 0) + (n > 32 ? (paged ? 3.5 : 4.5) * n : 0);
-    if (*nsplit && cost >= best) continue;
-    best = cost;
-    *nsplit = slices;
-    *split_len = (int)sl;
+  const auto consider = [&](int n) {
+    const unsigned sl = ((ucap + n - 1) / n + unit - 1) / unit * unit;
+    if (n > 1 && sl < 64) return false;
+    const int slices = (int)((ucap + sl - 1) / sl);
+    const double cost = (double)((segs * slices + slots - 1) / slots) * (double)(sl + 100) +
+                        (slices > 1 ? 75 : 0) +
+                        (slices > 32 ? (paged ? 3.5 : 4.5) * slices : 0);
+    if (!*nsplit || cost < best) {
+      best = cost;
+      *nsplit = slices;
+      *split_len = (int)sl;
+    }
+    return true;
+  };
+  // Launches plan too, so not every count up to 256 is looked at (9 us of host
+  // time): the small ones, then the most slices of each of the first rounds and
+  // 32, the sizes about which the cost turns.  Between those the cost falls with
+  // the count, but for more than 32 slices, whose own term grows: those in
+  // steps of an eighth.
+  int n = 1;
+  while (n <= 8 && consider(n)) ++n;
+  if (n <= 8) return;
+  for (int r = 1; r <= 8; ++r) {
+    const long long m = r * slots / segs;
+    if (m > 8 && m <= 256) consider((int)m);
+  }
+  consider(16);
+  consider(24);
+  for (n = 32; n <= 256 && consider(n); n += n / 8) {
   }
 }
 
@@ -199,13 +217,14 @@ static int decode_attention(const char* op, bool noalloc, const void* q, const v
                       (q_dtype == kv_dtype ? aligned16(q) : true));
   if (mfma) {
     int ns = 1, sl = 0;
-    plan_split(batch, q_heads, kv_heads, seq_len, p.page_size, paged, &ns, &sl);
-    if (!f32 && !noalloc && workspace && aligned16(workspace) &&
-        workspace_bytes >= tm_decode_attention_full_workspace_size(
-                               batch, q_heads, kv_heads, head_dim, seq_len,
-                               paged ? page_size : 0))
+    const size_t per = (size_t)batch * q_heads * (head_dim + 4) * sizeof(float);
+    bool full = !f32 && !noalloc && workspace && aligned16(workspace);
+    if (full) {
       plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged, &ns, &sl);
-    const size_t need = (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float);
+      full = ns == 1 || workspace_bytes >= per * ns;
+    }
+    if (!full) plan_split(batch, q_heads, kv_heads, seq_len, p.page_size, paged, &ns, &sl);
+    const size_t need = per * ns;
     if (noalloc && ns > 1) {
       static DeviceGlobal scratch("tm_decode_scratch");
       void* ptr = nullptr;
