@@ -258,3 +258,43 @@ def test_small_workspace_keeps_the_other_kernels():
         torch.cuda.synchronize()
         tol = 2.0 ** -11 * 1.01 * ref.abs() + _sum_bound(x, deq, mag) + 1e-6
         assert bool(((y.cpu().double() - ref).abs() <= tol).all()), nbytes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["int4", "decode", "kda"])
+def test_workspace_belongs_to_the_plans_stream(op):
+    """A plan bound to a stream other than the current one takes its workspace from
+    that stream's memory: not what the current stream freed a moment ago (its work
+    there may still run), and what a dropped plan gives back (its own work may still
+    run) does not go to the current stream's tensors.  Nothing is launched."""
+    side = torch.cuda.Stream()
+    zeros = lambda *s, dt=torch.float16: torch.zeros(*s, dtype=dt, device="cuda")
+    if op == "int4":
+        M, N, K = 300, 2816, 7040
+        a = [zeros(M, K), zeros(N, K // 2, dt=torch.uint8), zeros(M, N), zeros(N, K // 128)]
+        plan = lambda s: tm.plan_int4_matmul(*a, None, M, N, K, 128, stream=s)
+        ws = lambda p: p._keep
+    elif op == "decode":
+        q, kv = zeros(2, 8, 128), zeros(2, 8, 8192, 128)
+        o = torch.empty_like(q)
+        plan = lambda s: tm.plan_decode_attention(q, kv, kv, o, stream=s)
+        ws = lambda p: p._keep[1]
+    else:
+        bf = torch.bfloat16
+        q, g, b = zeros(1, 640, 4, 128, dt=bf), zeros(1, 640, 4, 128, dt=torch.float32), zeros(
+            1, 640, 4, dt=torch.float32)
+        o = torch.empty_like(q)
+        plan = lambda s: tm.plan_chunk_kda(q, q, q, g, b, o, stream=s)
+        ws = lambda p: p._keep
+    size = ws(plan(None)).numel()
+    freed = torch.empty(size, dtype=torch.uint8, device="cuda")
+    at = freed.data_ptr()
+    del freed
+    p = plan(side.cuda_stream)
+    w = ws(p)
+    assert w.numel() == size and w.data_ptr() != at
+    at = w.data_ptr()
+    del p, w
+    assert torch.empty(size, dtype=torch.uint8, device="cuda").data_ptr() != at
+    with torch.cuda.stream(side):
+        assert torch.empty(size, dtype=torch.uint8, device="cuda").data_ptr() == at

@@ -84,7 +84,9 @@ class Launch:
 
     Calling it launches asynchronously on the stream bound at creation (the
     current stream of the tensors' device then) or on ``stream`` if given.
-    The device must be the current HIP device when called."""
+    The device must be the current HIP device when called.  A workspace that
+    the plan allocated belongs to the stream bound at creation (_workspace):
+    keep the plan until another ``stream`` that ran it is done."""
 
     __slots__ = ("_f", "_args", "_what", "dev", "stream", "_keep")
 
@@ -100,6 +102,17 @@ class Launch:
         rc = self._f(*self._args, self.stream if stream is None else stream)
         if rc:
             _lib.check(rc, self._what, kernel_name=self._what)
+
+
+def _workspace(nbytes, dev, stream):
+    """nbytes of device memory for a plan on ``stream`` (None: the current one):
+    from the pool of that stream, so that what a dropped plan gives back is
+    handed out only behind its work there, and what was freed on the current
+    stream a moment ago is not handed to it."""
+    if stream is None or stream == _stream(dev):
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    with torch.cuda.stream(torch.cuda.ExternalStream(stream, device=dev)):
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
 
 
 def _run(launch: Launch):
@@ -190,12 +203,13 @@ def plan_int4_matmul(input, weight, output, scales, zeros, M, N, K, group_size=1
 def _wq_launch(qbits, input, weight, bias, output, scales, zeros, M, N, K, group_size, adt, sdt,
                zdt, what, dev, stream):
     """Bind a validated weight-only call to tm_wq_matmul_ws with the device
-    workspace its plan needs (split-K shapes; none otherwise), allocated here
-    from torch's caching allocator and kept alive with the launch."""
+    workspace its plan needs (split-K sums, the pipelined int4 kernels' copy of
+    the activations; often none), allocated here from torch's caching allocator
+    and kept alive with the launch."""
     L = _lib.lib()
     ws_bytes = L.tm_wq_workspace_bytes(qbits, _ptr(input), _ptr(weight), _ptr(scales),
                                        _ptr(zeros), M, N, K, group_size, adt, sdt, zdt)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    ws = _workspace(ws_bytes, dev, stream) if ws_bytes else None
     args = (qbits, _ptr(input), _ptr(weight), _ptr(bias), _ptr(output), _ptr(scales),
             _ptr(zeros), M, N, K, group_size, adt, sdt, zdt, _ptr(ws), ws_bytes)
     launch = Launch(L.tm_wq_matmul_ws, args, what, dev, stream)
@@ -842,7 +856,7 @@ def plan_decode_attention(q, k_cache, v_cache, o, seq_lens=None, seq_len=None, p
     need = _lib.lib().tm_decode_attention_full_workspace_size(
         B, Hq, Hkv, D, seq_len, page_size if page_table is not None else 0)
     if workspace is None and need > 0:
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+        workspace = _workspace(need, dev, stream)
     wbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     st = (C.c_longlong * 3)(*strides)
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(o), _ptr(lse), B, Hq, Hkv, D,
@@ -1045,7 +1059,7 @@ def plan_chunk_kda(q, k, v, g, beta, o, scale=None, initial_state=None, final_st
         raise ValueError(f"unsupported KDA shape: key_dim={Dk} value_dim={Dv} "
                          f"chunk_size={chunk_size} (supported: 128, 128, 64)")
     if workspace is None:
-        workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+        workspace = _workspace(max(need, 16), dev, stream)
     elif workspace.numel() * workspace.element_size() < need:
         raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} "
                          f"bytes, needs {need}")
