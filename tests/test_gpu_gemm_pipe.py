@@ -95,6 +95,78 @@ def test_every_kernel(kind, layout, tile):
         _close(C, ref, bound + 2 * U[torch.float32] * ref.abs(), odt)
 
 
+def _unaligned(b, rows, cols, dt, transposed, seed, off=1):
+    """[b, rows, cols] of small random values without any padding: the first
+    element `off` past an aligned address, one element (NaN) between the batches
+    and after the last."""
+    g = torch.Generator().manual_seed(seed)
+    d0, d1 = (cols, rows) if transposed else (rows, cols)
+    step = d0 * d1 + 1
+    flat = torch.full((off + b * step,), float("nan")).to(dt)
+    for i in range(b):
+        flat[off + i * step:][:d0 * d1] = torch.randn(d0 * d1, generator=g).to(dt)
+    t = flat.cuda().as_strided((b, d0, d1), (step, d1, 1), off)
+    return t.transpose(1, 2) if transposed else t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("layout", ["kk", "kr", "rk", "rr"])
+@pytest.mark.parametrize("kind", KINDS)
+def test_every_kernel_fills_by_elements(kind, layout, tile):
+    """The pieces that no copy may take whole (MmParams::fix, as mm_plan sets it for
+    operands like these), in the only k step and in the last of several: K no whole
+    number of pieces, row-contiguous rows that end inside one, an odd batch stride."""
+    from triton_metal_amd import _lib
+    from triton_metal_amd.driver import HipUtils
+    hu = HipUtils()
+    rt, ct = TILES[tile]
+    bm, bn, dt = 64 * rt, 64 * ct, KINDS[kind]
+    al, bk = (16, 128) if dt.itemsize == 1 else (8, 64)
+    fn = hu.builtin_function(f"mm_{kind}_{layout}_{tile}")
+    ar, br = layout[0] == "r", layout[1] == "r"
+    for i, (M, N, K) in enumerate(((bm + 5, bn - 3, 2 * bk + al // 2 + 1), (bm - 1, bn + 9, al - 1),
+                                   (al + 3, 2 * bn + 1, 4 * bk + 1), (bm + 1, al + 7, bk - 3),
+                                   (bm, bn, 3 * bk))):
+        b = 1 + i % 2
+        A = _unaligned(b, M, K, dt, ar, 3 * i)
+        B = _unaligned(b, K, N, dt, not br, 3 * i + 1)
+        C = torch.full((b, M, N), float("nan"), device="cuda")
+        p = Params(A.data_ptr(), B.data_ptr(), C.data_ptr(), None)
+        p.sa_b, p.sb_b, p.sc_b = A.stride(0), B.stride(0), C.stride(0)
+        p.sc_m, p.sc_n, p.M, p.N, p.K = N, 1, M, N, K
+        p.lda, p.ldb = A.stride(2 if ar else 1), B.stride(1 if br else 2)
+        p.tiles_m, p.tiles_n = -(-M // bm), -(-N // bn)
+        p.out_dt = DTC[torch.float32]
+        p.fix = (4 if ar else 1 if K % al else 0) | (8 if br else 2 if K % al else 0)
+        args = (ctypes.c_void_p * 1)(ctypes.cast(ctypes.pointer(p), ctypes.c_void_p))
+        rc = hu._lib.tm_launch(fn, p.tiles_m * p.tiles_n, b, 1, 256, 1, 1, 0,
+                               torch.cuda.current_stream().cuda_stream, args)
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        ref = A.double() @ B.double().contiguous()
+        bound = K * U[torch.float32] * (A.double().abs() @ B.double().abs().contiguous())
+        _close(C, ref, bound, torch.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("M,N,K", [(72, 136, 208), (300, 520, 1040)])
+def test_odd_batch_stride(dt, M, N, K):
+    """tm.dot on batches of aligned rows whose batch stride alone is odd."""
+    for ta in (False, True):
+        for tb in (False, True):
+            a = _unaligned(3, M, K, dt, ta, 1, off=0)
+            b = _unaligned(3, K, N, dt, tb, 2, off=0)
+            c = torch.full((3, M, N), 7.0, device="cuda")
+            tm.dot(a, b, c)
+            torch.cuda.synchronize()
+            ref = a.double().contiguous() @ b.double().contiguous()
+            bound = K * U[torch.float32] * (a.double().abs().contiguous()
+                                            @ b.double().abs().contiguous())
+            _close(c, ref, bound, torch.float32)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", KINDS.values(), ids=KINDS)
 @pytest.mark.parametrize("M,N,K", [(5, 70, 33), (129, 257, 131), (64, 33, 1), (300, 190, 1027),
