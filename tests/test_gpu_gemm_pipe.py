@@ -241,11 +241,12 @@ def test_selection():
     """Which sizes take the pipelined kernels and which keep the others, and
     the layouts and alignments they refuse (no device is touched)."""
     k = lambda *a, **kw: tm.gemm_kernel_for(*a, **kw)[0]
-    assert k(4096, 4096, 4096) == "mm_f16_kr_44"
+    assert k(4096, 4096, 4096) == "gemm_t256_nn_f16_same"
+    assert k(2048, 11008, 4096) == "mm_f16_kr_42" and k(4096, 4352, 4096)[:9] == "mm_f16_kr"
     assert k(4096, 4096, 4096, trans_b=True, in_dtype=torch.bfloat16) == "mm_bf16_kk_44"
     assert k(16, 11008, 4096, trans_b=True, bias=True) == "mm_f16_kk_11"
     assert k(2000, 11008, 4096, trans_b=True) == "mm_f16_kk_42"
-    assert {k(M, 4096, 4096)[-2:] for M in (64, 512, 1024, 2048, 4096)} >= {"11", "44"}
+    assert {k(M, 4096, 4096, trans_b=True)[-2:] for M in (64, 512, 1024, 2048, 4096)} >= {"11", "44"}
     # odd N is fine for [N, K] weights, not for rows of [K, N]
     assert k(300, 1001, 1024, trans_b=True).startswith("mm_f16_kk_")
     assert k(300, 1001, 1024) == "tm_dot"
@@ -253,3 +254,17 @@ def test_selection():
     assert k(300, 1000, 1024, lda=1028) == "tm_dot"
     assert k(512, 512, 512).startswith("gemm_s32k128_")
     assert k(4096, 4096, 64).startswith("gemm_t256_")
+    # 256-tile problems on both sides of its rules (rounds of CUs filled; K)
+    t256 = lambda *a, **kw: k(*a, **kw).startswith("gemm_t256_")
+    assert not t256(2048, 4096, 1024) and t256(2304, 4096, 1024) and t256(2304, 4096, 4096)
+    assert not t256(4096, 5120, 1024) and t256(5120, 5120, 1024) and not t256(5120, 5120, 4096)
+    assert t256(8192, 4096, 4096) and not t256(8192, 4096, 4096 + 32) and not t256(8192, 4095, 4096)
+    assert t256(3584, 4096, 3072, trans_b=True) and not t256(3584, 4096, 4096, trans_b=True)
+    # few rows of [N, K] weights, and the K-split kernel past two workgroups a CU
+    assert k(4, 8192, 384, trans_b=True).startswith("gemm_t32k_")
+    assert k(4, 16384, 384, trans_b=True).startswith("mm_") and k(33, 8192, 384, trans_b=True)[:3] == "mm_"
+    assert k(100, 2048, 648, trans_b=True).startswith("gemm_t32_")
+    assert k(128, 2048, 1152, trans_b=True).startswith("mm_") and k(100, 2048, 648).startswith("mm_")
+    assert k(16, 768, 1536, trans_b=True).startswith("gemm_t32_")
+    assert k(1024, 1024, 256).startswith("gemm_s32k64_") and k(4096, 256, 256).startswith("mm_")
+    assert k(768, 768, 512).startswith("gemm_s32k128_") and k(1024, 768, 512).startswith("mm_")

@@ -503,19 +503,46 @@ void gemm_plan(int M, int N, int K, int lda, int ldb, int ldc, bool bt, bool bia
     const long t32s = (M % 32 == 0 && N % 32 == 0) ? (long)(M / 32) * (N / 32) : 0;
     const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
     const long t256 = (M % 256 == 0 && N % 256 == 0) ? (long)(M / 256) * (N / 256) : 0;
-    // The pipelined kernels (gemm_pipe.h), except where there is too little to
-    // pipeline (us here / there, bf16, one box): one k step (K <= 64: 1024 x 832
-    // 3.4 / 3.3, 4096 x 4096 12.1 / 12.8); two of them with weights [N, K]
+    // 256 x 256 tiles (gemm_big.hip), one workgroup per CU, for aligned problems
+    // from 32 tiles on whose 32-bit copy offsets fit (up to 256 rows of A / B^T,
+    // 64 rows of B)
+    const bool can256 = t256 >= 32 && K % 64 == 0 && 256LL * lda * 2 < (1LL << 32) &&
+                        (bt ? 256LL : 64LL) * ldb * 2 < (1LL << 32);
+    // ... before the pipelined kernels where its rounds of tiles leave few CUs idle:
+    // its tile starts and ends in 3 us less and its k step is as long, so short K
+    // gains most (us, 256 tiles / pipelined, nn; share of the rounds' CUs busy):
+    //   3328 x 4096 (.81) K = 256 14.5 / 21.3, 1024 30.6 / 38.2, 4096 103 / 105
+    //   2304 x 4096 (.56) K = 256 13.0 / 16.5, 1024 26.3 / 32.5, 4096 85 / 90
+    //   2048 x 4096 (.50) K = 256 13.7 / 12.9, 1024 28.3 / 24.5, 4096 80 / 68
+    //   4096 x 4096 (1) K = 512 22.1 / 28.6, 2048 57.3 / 63.4, 4096 119 / 119
+    //   6144 x 5120 (.94) K = 1024 67 / 77, 3072 170 / 169; 8192 x 8192 (1) K = 1024
+    //   141 / 158, 2048 251 / 262; 5120 x 5120 (.78) K = 2048 103 / 111, 4096 212 /
+    //   218; 7168 x 5120 (.73) K = 1024 96 / 90, 3072 238 / 228; nt 3584 x 4096 (.88)
+    //   K = 3072 79 / 84, 4096 107 / 102, 4096 x 4096 x 4096 111 / 109
+    const long rounds = (t256 + 255) / 256;
+    const bool big256 = can256 && (rounds == 1  ? t256 >= 141 && !(bt && K >= 4096 && t256 >= 200)
+                                   : K <= 2048 ? 100 * t256 >= 78 * 256 * rounds
+                                               : t256 == 256 * rounds);
+    // The other sizes take the pipelined kernels (gemm_pipe.h), except where there
+    // is too little to pipeline (us here / there, bf16, one box): one k step (K <= 64:
+    // 1024 x 832 3.4 / 3.3, 4096 x 4096 12.1 / 12.8); two of them with weights [N, K]
     // (K <= 128: 1136 x 1968 5.2 / 5.5; nn 6.7 / 5.7) or on 256-tile problems
     // (4096 x 4096 near even); the K-split kernel's sizes up to two workgroups
-    // a CU (256 x 512 x 512 2.9 / 4.5; past it 1024 x 1024 x 512 5.8 / 4.9, 2048
-    // x 1920 x 256 10.5 / 6.8); up to 64 tiles with K staged at once (500 x 500
-    // x 504 4.1 / 4.9, past it 800 x 800 x 512 9.0 / 4.9); and outputs of four
-    // tiles or fewer (100 x 72 x 1000 nt 6.9 / 8.2, nn 15 / 8.7).
-    const bool s32k = t32s > 0 && t32s <= 512 && (K == 256 || K == 512) && c16 && ldc % 4 == 0;
-    const bool small = K <= 64 || (K <= 128 && (bt || t256 >= 32)) || s32k ||
+    // a CU, and compact ones somewhat past it (256 x 512 x 512 2.9 / 4.5, 768 x 768
+    // x 512 5.8 / 6.3, 1024 x 768 x 512 6.6 / 6.3; 1024 x 1024 x 256 4.5 / 5.2, 1280
+    // x 1280 x 256 6.4 / 6.4, 4096 x 256 x 256 6.2 / 5.1); up to 64 tiles with K staged
+    // at once (500 x 500 x 504 4.1 / 4.9, past it 800 x 800 x 512 9.0 / 4.9) or 32 rows
+    // of [N, K] weights and 128 (4 x 8192 x 384 4.3 / 5.1, 4 x 16384 6.9 / 5.4); up to
+    // 64 tiles of [N, K] weights to K = 1024 (100 x 2048 x 648 5.6 / 6.1, past it 128
+    // x 2048 x 1152 10.5 / 7.9), 16 to 1536 (16 x 768 x 1536 9.5 / 9.9); and
+    // outputs of four tiles or fewer (100 x 72 x 1000 nt 6.9 / 8.2, nn 15 / 8.7).
+    const bool s32k = t32s > 0 && c16 && ldc % 4 == 0 && (K == 256 || K == 512) &&
+                      (t32s <= 512 || (t32s <= (K == 256 ? 1024 : 576) && M <= 1024 && N <= 1024));
+    const bool few = bt && ((t64 <= 128 && M <= 32 && K <= 512) || (t64 <= 64 && K <= 1024) ||
+                            (t64 <= 16 && K <= 1536));
+    const bool small = K <= 64 || (K <= 128 && (bt || t256 >= 32)) || s32k || few ||
                        (t64 <= 64 && K <= 512) || (t64 <= 4 && K <= 1024);
-    if (!small) {
+    if (!small && !big256) {
       // pointers only as aligned as the caller said
       const void* al = (const void*)16;
       const MmCall c = mm_call(al, al, (void*)16, bias ? al : nullptr, M, N, K, lda, ldb, ldc,
@@ -528,14 +555,9 @@ void gemm_plan(int M, int N, int K, int lda, int ldb, int ldc, bool bt, bool bia
         return;
       }
     }
-    // 256 x 256 tiles (gemm_big.hip) for aligned problems from 32 tiles on:
-    // one such workgroup per CU beats four 128 x 128 ones over the same
-    // outputs even when most CUs stay idle (one box, fp16, K = 4096: 2048 x
-    // 3072 78 against 125 us, 2560 x 4096 84 against 241; at 16 tiles the
-    // smaller tiles win, 140 against 147 us); the 32-bit copy offsets of a
-    // tile (up to 256 rows of A / B^T, 64 rows of B) must fit
-    if (t256 >= 32 && K % 64 == 0 && 256LL * lda * 2 < (1LL << 32) &&
-        (bt ? 256LL : 64LL) * ldb * 2 < (1LL << 32)) {
+    // (the short K that is left: one workgroup per CU beats four 128 x 128 ones over
+    // the same outputs even when most CUs stay idle)
+    if (can256) {
       snprintf(pl->name, sizeof pl->name, "gemm_t256_%s_%s_%s%s", bt ? "nt" : "nn", dt, od, bs);
       pl->grid = (unsigned)t256;
       pl->block = 512;

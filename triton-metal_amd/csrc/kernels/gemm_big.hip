@@ -4,7 +4,8 @@
 //   C[M, N] = A[M, K] @ W[N, K]^T (+ bias[N])  (nt: the nn.Linear layout)
 //
 // for M % 256 == 0, N % 256 == 0, K % 64 == 0 (the host picks it for large
-// aligned problems of at most 128 k; the others run in gemm_pipe.h or gemm.hip).  Reference semantics as
+// aligned problems whose tiles fill their rounds of CUs, and for short K; the others
+// run in gemm_pipe.h or gemm.hip).  Reference semantics as
 // gemm.hip: make_matmul_kernel / make_simdgroup_matmul_kernel /
 // make_fused_linear_kernel (_msl_templates.py:447-585, 3501-3667, 4013-4135).
 //
