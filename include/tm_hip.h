@@ -383,6 +383,16 @@ int tm_kda_chunk_fwd(const void* q, const void* k, const void* v, const float* g
                      int batch, int seq_len, int heads, int key_dim, int value_dim,
                      int chunk_size, float scale, int beta_dtype, void* workspace,
                      size_t workspace_bytes, void* stream);
+/* tm_kda_chunk_fwd for a workspace that no other call shares: at least
+ * tm_kda_compact_workspace_size(...) bytes (never more than the size above; long
+ * sequences pass through one smaller place in segments). The same results. */
+size_t tm_kda_compact_workspace_size(int batch, int seq_len, int heads, int key_dim, int value_dim,
+                                     int chunk_size);
+int tm_kda_chunk_fwd_compact(const void* q, const void* k, const void* v, const float* g,
+                             const void* beta, const float* initial_state, void* o,
+                             float* final_state, int batch, int seq_len, int heads, int key_dim,
+                             int value_dim, int chunk_size, float scale, int beta_dtype,
+                             void* workspace, size_t workspace_bytes, void* stream);
 /* The same rule token by token (the recurrent form; no counterpart in the
  * reference either): for decoding one or a few tokens that continue from a
  * state, e.g. the final_state of tm_kda_chunk_fwd.  Arguments as

@@ -99,6 +99,32 @@ def test_kda_workspace_and_validation():
                                 None) == 0
 
 
+def test_kda_compact_workspace():
+    """A workspace that no other call shares: one place of at most 1700 chunks, and the
+    state handed on, for more than 2000 chunks; never more than the shared one's size."""
+    import triton_metal_amd as tm
+    import triton_metal_amd._lib as L
+    lib = L.lib()
+    size = lambda B, T, H: lib.tm_kda_compact_workspace_size(B, T, H, 128, 128, 64)
+    for B, T, H, seg in ((1, 6200, 16, 97), (3, 2048, 20, 32), (1, 8000, 16, 125),  # one pass
+                         (1, 8192, 16, 64), (2, 4096, 24, 32), (1, 16384, 16, 86),
+                         (4, 8192, 16, 26), (1, 131072, 1, 1024), (1, 1 << 20, 1, 1639)):
+        nc, bh = -(-T // 64), B * H
+        state = 0 if seg == nc else 4 * 128 * 128
+        assert size(B, T, H) == bh * (seg * 74240 + state) <= tm.kda_workspace_size(B, T, H)
+        assert seg == nc <= 2000 // bh or seg * bh <= 1700 + bh
+    # segments of fewer than 4 chunks are not made
+    assert size(16, 1024, 32) == tm.kda_workspace_size(16, 1024, 32)
+    assert size(1, 64, 0) == size(0, 64, 4) == size(1, 0, 4) == 0
+    assert lib.tm_kda_compact_workspace_size(1, 8192, 16, 64, 128, 64) == 0
+    p = ctypes.c_void_p(16)
+    args = [p, p, p, p, p, None, p, None, 1, 8192, 16]
+    call = lambda *a: lib.tm_kda_chunk_fwd_compact(*args, *a, None)
+    assert call(64, 128, 64, 0.1, L.TM_DT_F32, p, 1 << 30) == L.TM_ERR_UNSUPPORTED
+    assert call(128, 128, 64, 0.1, L.TM_DT_F32, p, size(1, 8192, 16) - 1) == L.TM_ERR_INVALID_ARG
+    assert "tm_kda_chunk_fwd_compact: workspace" in L.last_error()
+
+
 def test_int8_matmul_rejects_uint8_weights():
     """The kernels read the weight bytes as signed int8 (the reference's
     `device const char*`); uint8 storage is refused rather than misread."""

@@ -343,19 +343,33 @@ def test_kda_graph_replays_track_new_inputs(dev):
 
 
 @pytest.mark.gpu
-def test_kda_segments_match_separate_calls():
-    """Enough chunks that one call walks the sequence in segments (1846 chunks:
-    two of 36 and 35 chunks a head, the last one partial): the same bits as two
-    calls cut elsewhere with the state handed over."""
-    B, T, H = 2, 64 * 70 + 5, 13
+@pytest.mark.parametrize("B,T,H,shared", [(2, 64 * 70 + 5, 15, False), (1, 64 * 40, 100, False),
+                                          (2, 64 * 70 + 5, 23, True)])
+def test_kda_segments_match_separate_calls(B, T, H, shared):
+    """Enough chunks that one call walks the sequence in segments (more than 2000 in a
+    plan's own workspace, 3072 in a shared one; the last segment shorter, its last chunk
+    partial): the same bits as two shorter calls in one pass each with the state
+    handed over."""
     q, k, v, g, beta = (t.cuda() for t in kda_inputs(B, T, H, seed=9))
     s0 = 0.1 * torch.randn(B, H, 128, 128, generator=torch.Generator().manual_seed(1)).cuda()
-    o, st = tm.chunk_kda(q, k, v, g, beta, initial_state=s0, output_final_state=True)
-    o_only, none = tm.chunk_kda(q, k, v, g, beta, initial_state=s0)
-    cut = 64 * 50
+    full, compact = (f(B, T, H, 128, 128, 64) for f in (tm._lib.lib().tm_kda_workspace_size,
+                                                        tm._lib.lib().tm_kda_compact_workspace_size))
+    assert compact < full
+    ws = torch.empty(full, dtype=torch.uint8, device="cuda") if shared else None
+    outs = []
+    for want_state in (True, False):
+        o = torch.full_like(v, float("nan"))
+        st = torch.full_like(s0, float("nan")) if want_state else None
+        plan = tm.plan_chunk_kda(q, k, v, g, beta, o, initial_state=s0, final_state=st, workspace=ws)
+        assert shared or plan._keep.numel() == compact
+        plan()
+        outs.append((o, st))
+    (o, st), (o_only, _) = outs
+    cut = 64 * 20
     first, rest = ([t[:, :cut].contiguous() for t in (q, k, v, g, beta)],
                    [t[:, cut:].contiguous() for t in (q, k, v, g, beta)])
     o1, mid = tm.chunk_kda(*first, initial_state=s0, output_final_state=True)
     o2, end = tm.chunk_kda(*rest, initial_state=mid, output_final_state=True)
-    assert none is None and torch.equal(o, o_only)
+    assert B * H * (-(-T // 64) - 20) <= 3072  # one pass
+    assert torch.equal(o, o_only)
     assert torch.equal(o, torch.cat((o1, o2), 1)) and torch.equal(st, end)

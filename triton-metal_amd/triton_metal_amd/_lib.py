@@ -66,6 +66,7 @@ SIGNATURES = {
     "tm_flash_attention": [vp, vp, vp, vp, vp, i32, i32, i32, i32, C.POINTER(C.c_longlong),
                            C.c_float, i32, i32, vp],
     "tm_kda_workspace_size": [i32, i32, i32, i32, i32, i32],
+    "tm_kda_compact_workspace_size": [i32, i32, i32, i32, i32, i32],
     "tm_decode_attention_workspace_size": [i32, i32, i32, i32, i32, i32],
     "tm_decode_attention_full_workspace_size": [i32, i32, i32, i32, i32, i32],
     "tm_decode_attention": [vp, vp, vp, vp, vp, i32, i32, i32, i32, vp, i32,
@@ -76,6 +77,8 @@ SIGNATURES = {
                                     i32, vp],
     "tm_kda_chunk_fwd": [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, C.c_float,
                          i32, vp, sz, vp],
+    "tm_kda_chunk_fwd_compact": [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32,
+                                 C.c_float, i32, vp, sz, vp],
     "tm_kda_recurrent_fwd": [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, C.c_float,
                              i32, vp],
 }
@@ -84,6 +87,7 @@ _RESTYPES = {
     "tm_version": C.c_char_p,
     "tm_builtin_module_name": C.c_char_p,
     "tm_kda_workspace_size": sz,
+    "tm_kda_compact_workspace_size": sz,
     "tm_decode_attention_workspace_size": sz,
     "tm_decode_attention_full_workspace_size": sz,
     "tm_wq_workspace_bytes": sz,

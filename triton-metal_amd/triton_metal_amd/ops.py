@@ -1051,14 +1051,18 @@ def plan_chunk_kda(q, k, v, g, beta, o, scale=None, initial_state=None, final_st
     q, k: bf16 [B, T, H, 128]; v, o: bf16 [B, T, H, 128]; g: fp32 [B, T, H, 128]
     (log decay); beta: fp32 or bf16 [B, T, H]; initial_state / final_state:
     fp32 [B, H, 128, 128] or None; workspace: a uint8 device tensor of at least
-    kda_workspace_size(B, T, H) bytes (allocated here when None)."""
+    kda_workspace_size(B, T, H) bytes, which calls may share one after the other
+    (None: the plan's own is allocated here, a smaller one for long sequences)."""
     dev, B, T, H, Dk, Dv = _kda_check(q, k, v, g, beta, o, initial_state, final_state,
                                       workspace)
-    need = _lib.lib().tm_kda_workspace_size(B, T, H, Dk, Dv, chunk_size)
+    L = _lib.lib()
+    own = workspace is None
+    need = (L.tm_kda_compact_workspace_size if own else L.tm_kda_workspace_size)(
+        B, T, H, Dk, Dv, chunk_size)
     if need == 0 and B * T * H > 0:
         raise ValueError(f"unsupported KDA shape: key_dim={Dk} value_dim={Dv} "
                          f"chunk_size={chunk_size} (supported: 128, 128, 64)")
-    if workspace is None:
+    if own:
         workspace = _workspace(max(need, 16), dev, stream)
     elif workspace.numel() * workspace.element_size() < need:
         raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} "
@@ -1069,7 +1073,8 @@ def plan_chunk_kda(q, k, v, g, beta, o, scale=None, initial_state=None, final_st
     args = (_ptr(q), _ptr(k), _ptr(v), _ptr(g), _ptr(beta), _ptr(initial_state), _ptr(o),
             _ptr(final_state), B, T, H, Dk, Dv, chunk_size, float(scale), bdt, _ptr(workspace),
             workspace.numel() * workspace.element_size())
-    launch = Launch(_lib.lib().tm_kda_chunk_fwd, args, "kda_chunk_fwd", dev, stream)
+    launch = Launch(L.tm_kda_chunk_fwd_compact if own else L.tm_kda_chunk_fwd, args,
+                    "kda_chunk_fwd", dev, stream)
     launch._keep = workspace
     return launch
 
@@ -1119,6 +1124,9 @@ def chunk_kda(q, k, v, g, beta, scale=None, initial_state=None, output_final_sta
     o = torch.empty(B, T, H, Dv, dtype=torch.bfloat16, device=q.device)
     st = (torch.empty(B, H, Dk, Dv, dtype=torch.float32, device=q.device)
           if output_final_state else None)
+    # the caching allocator hands calls one after the other the same workspace
+    ws = torch.empty(max(16, kda_workspace_size(B, T, H, Dk, Dv, chunk_size)), dtype=torch.uint8,
+                     device=q.device)
     _run(plan_chunk_kda(q, k, v, g, beta, o, scale=scale, initial_state=initial_state,
-                        final_state=st, chunk_size=chunk_size))
+                        final_state=st, workspace=ws, chunk_size=chunk_size))
     return o, st
