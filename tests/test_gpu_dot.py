@@ -117,6 +117,38 @@ def test_dot_column_major_output(dev, dt):
     _check(cbuf.t(), oracle.dot(_np(a), _np(b)), dt, np.abs(_np(a)), np.abs(_np(b)))
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("batch,M,N,K", [(1, 72, 136, 40), (2, 200, 64, 272), (1, 2504, 2496, 80),
+                                         (3, 1160, 2056, 136)])
+def test_dot_column_major_output_tiles(dev, dt, ta, tb, batch, M, N, K):
+    """Outputs that are not row-contiguous stay on the dot_tile kernels: each operand k-
+    or row-contiguous in 16-byte pieces, 64 x 64 tiles (the first two sizes) and 128 x
+    128 ones, against the product in 64 bits: |err| <= one rounding + K u sum |a||b|."""
+    al = 16 // dt.itemsize
+    M, N, K = (-(-d // al) * al for d in (M, N, K))
+    g = torch.Generator().manual_seed(M + N + K)
+
+    def operand(rows, cols, t):
+        x = torch.randn(batch, *((cols, rows) if t else (rows, cols)), generator=g).to(dt).to(dev)
+        return x.transpose(1, 2) if t else x
+
+    a, b = operand(M, K, ta), operand(K, N, tb)
+    odt = torch.float32 if dt.itemsize == 1 else dt
+    z = torch.randn(batch, N, M, generator=g).to(odt).to(dev).transpose(1, 2)
+    ad, bd = a.double().contiguous(), b.double().contiguous()
+    ref, mag = ad @ bd, ad.abs() @ bd.abs()
+    u = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[odt]
+    for epilogue in ("none", "add-matrix"):
+        c = torch.full((batch, N, M), float("nan"), dtype=odt, device=dev).transpose(1, 2)
+        add = epilogue == "add-matrix"
+        tm.dot(a, b, c, epilogue, z=z if add else None)
+        want = ref + z.double() if add else ref
+        tol = 1.01 * u * want.abs() + (K + 2) * 2.0 ** -24 * (mag + want.abs())
+        err = (c.double() - want).abs()
+        assert bool((err <= tol).all()), float((err / tol).max())
+
+
 @pytest.mark.parametrize("layout", ["row", "trans_a", "trans_b", "strided"])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
 def test_dot_batched_3d(dev, layout, dt):

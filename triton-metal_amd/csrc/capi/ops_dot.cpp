@@ -215,8 +215,11 @@ int dot_impl(const char* op, const void* A, const void* B, void* C, const void* 
       if (used || rc) return rc;
     }
   }
-  // 16-bit and e4m3 / e5m2 operands in aligned 16-byte pieces along k or along
-  // the rows, any batch and add epilogue: the pipelined kernels
+  // 16-bit and e4m3 / e5m2 operands contiguous along k or along the rows at any
+  // alignment, rows of C contiguous, any batch and add epilogue: the pipelined
+  // kernels, at every size (420 calls of 1 to 64 batches, 16 to 2048 rows and K from 8
+  // in all layouts: 0.54 of the dot_tile kernels' time in the geometric mean, none
+  // slower; 16 batches of 64 x 64 x 64 e4m3 7.2 -> 4.4 us)
   if (!rows_kernel && (epilogue == TM_EPI_NONE || add)) {
     MmCall c = {A, B, add ? Z : nullptr, C, batch, M, N, K,
                 st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7], st[8],
