@@ -336,6 +336,11 @@ size_t tm_decode_attention_workspace_size(int batch, int q_heads, int kv_heads, 
  * best (a smaller one: as above); never less than the size above. */
 size_t tm_decode_attention_full_workspace_size(int batch, int q_heads, int kv_heads,
                                                int head_dim, int seq_len, int page_size);
+/* The slices of one (sequence, KV head) that 16-bit caches take with that workspace,
+ * and the positions of each (own_lengths: at most, with seq_lens).  A diagnostic: touches
+ * no device. */
+int tm_decode_attention_plan(int batch, int q_heads, int kv_heads, int head_dim, int seq_len,
+                             int page_size, int own_lengths, int* slices, int* slice_positions);
 int tm_decode_attention(const void* q, const void* k_cache, const void* v_cache, void* o,
                         float* lse, int batch, int q_heads, int kv_heads, int head_dim,
                         const int* seq_lens, int seq_len, const long long* kv_strides,

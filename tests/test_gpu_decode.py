@@ -332,3 +332,51 @@ def test_paged_slices_past_64_pages(page_size, S):
         # P and O round to fp16: 2^-11 of the weighted sum of |V| each
         tol = 2.0 ** -10 * (p.unsqueeze(-1) * v.abs().unsqueeze(1)).sum(2).reshape(ref.shape)
         assert bool(((o[b].float() - ref).abs() <= tol + 1e-4).all()), (b, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,dt", [(64, torch.bfloat16), (128, torch.float16), (80, torch.float16)])
+@pytest.mark.parametrize("page", [0, 5, 48, 64])
+def test_each_sequence_is_cut_at_its_own_length(page, D, dt):
+    """Several slices per sequence whose lengths run from none to the capacity, on both
+    sides of the edges of its own slices (32 positions, whole pages), against the
+    softmax in 64 bits: the probabilities and the result round to 16 bits."""
+    Hkv, rep, S = 2, 4, 3000
+    lens = [0, 1, 31, 32, 33, 95, 97, 240, 241, 960, 961, 1499, 2999, 3000]
+    B = len(lens)
+    g = torch.Generator().manual_seed(page + D)
+    q = torch.randn(B, Hkv * rep, D, generator=g).to(dt).cuda()
+    kv = [torch.randn(B, Hkv, S, D, generator=g).to(dt) for _ in range(2)]
+    table = None
+    if page:
+        per = -(-S // page)
+        table = torch.randperm(B * per, generator=g).int().reshape(B, per)
+        paged = []
+        for t in kv:  # [pages, page, Hkv, D], NaN where no position is
+            pool = torch.full((B * per, page, Hkv, D), float("nan"), dtype=dt)
+            rows = torch.full((B, per * page, Hkv, D), float("nan"), dtype=dt)
+            rows[:, :S] = t.transpose(1, 2)
+            pool[table.long()] = rows.reshape(B, per, page, Hkv, D)
+            paged.append(pool.cuda())
+        kc, vc = paged
+        table = table.cuda()
+    else:
+        kc, vc = (t.cuda() for t in kv)
+    n = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    o = torch.full_like(q, float("nan"))
+    lse = torch.empty(B, Hkv * rep, device="cuda")
+    tm.plan_decode_attention(q, kc, vc, o, seq_lens=n, seq_len=S, page_table=table, lse=lse)()
+    u = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    for b, m in enumerate(lens):
+        k, v = (t[b, :, :m].double().cuda() for t in kv)
+        qb = q[b].double().reshape(Hkv, rep, D)
+        if m == 0:
+            assert bool((o[b] == 0).all()) and bool((lse[b] == float("-inf")).all())
+            continue
+        sc = (qb.unsqueeze(2) * k.unsqueeze(1)).sum(-1) * D ** -0.5
+        p = torch.softmax(sc, -1)
+        ref = (p @ v).reshape(Hkv * rep, D)
+        # |err| <= u (the result) + 2 u sum p |v| (each probability rounds once)
+        tol = 1.01 * u * ref.abs() + 2 * u * (p @ v.abs()).reshape(Hkv * rep, D) + 1e-6
+        assert bool(((o[b].double() - ref).abs() <= tol).all()), m
+        assert torch.allclose(lse[b].double(), torch.logsumexp(sc, -1).reshape(-1), atol=2e-3)

@@ -30,6 +30,7 @@ struct DecodeParams {
   int page_size, max_pages;
   int page_shift;
   int nsplit, split_len;
+  int slice_unit;
   float sl2;
   int q_dt, kv_dt, o_dt;
 };
@@ -73,18 +74,20 @@ void plan_split(int batch, int q_heads, int kv_heads, int cap, int page_size, bo
 // contiguous): 100 for its start, 75 for the combining launch, and where that has
 // more slices than the 32 it merges at once 0.2 us for each of them (us, one
 // sequence of 8192 positions, 1 KV head: 32 slices 23.4, 40 29.4, 64 26.7; 8 heads 24.4,
-// 31.4, 29.6; of 32768, 8 heads: 32 slices 74, 64 60, 96 58).  Every sequence counts as full, also with seq_lens: the host
-// does not know the lengths, and a count made for shorter ones starts a second
-// round when they are not.  us for lengths all full / from a quarter of the
-// capacity to all of it / all a quarter, and the slices: 16 sequences of 8 KV heads,
-// 8192 in 16-position pages, the plan above 150 / 146 / 143 (8), made for two
-// thirds 165 / 95 / 92 (7), here 108 / 103 / 95 (6); 32 of 8, 4096 152 / 146 / 144 (4),
-// 137 / 97 / 57 (11), 112 / 103 / 73 (3); 17 of 8, 16384, D = 64 120 / 110 / 107 (16), 127
-// / 78 / 65, 98 / 86 / 80 (11); 45 of 4, 4494 in 64-position pages 132 / 78 / 75 (5),
-// 134 / 80 / 76 (5), 95 / 88 / 87 (4): an odd count spreads the empty slices better
-// over the XCDs, which take workgroups in turn.
+// 31.4, 29.6; of 32768, 8 heads: 32 slices 74, 64 60, 96 58).
+// With lengths of their own (lens), every sequence is cut into that many slices of its
+// own length (slice_len in decode_attn.hip).  The host does not know the lengths: it
+// counts the rounds of full ones, where a round that is not filled costs most, and
+// a quarter of the longest slice on top, because in one round the longest
+// sequence's waves run alone at the end.  That takes two rounds from 64 (sequence, KV
+// head) pairs or so.  us all full / from a quarter of the capacity to all of it / all
+// a quarter: 16 sequences of 8 KV heads, 8192 in 16-position pages: the plan above 152 /
+// 149 / 143, one round 113 / 106 / 37, two 120 / 97 / 42, four 125 / 94 / 46; 32 of 8, 4096
+// 112 / 107 / 71, 113 / 106 / 39, 119 / 102 / 42, 126 / 92 / 43; 17 of 8, 16384, D = 64 126 /
+// 116 / 106, 96 / 81 / 32, 99 / 75 / 37, 112 / 84 / 42; 4 of 8, 32768 155 / 152 / 145, 114 / 109 /
+// 38 (taken), 133 / 108 / 54, 145 / 115 / 66.
 void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, int page_size,
-                 bool paged, int* nsplit, int* split_len) {
+                 bool paged, bool lens, int* nsplit, int* split_len) {
   const int group = q_heads / kv_heads, hbn = (group + 15) / 16;
   const long long segs = (long long)batch * kv_heads * hbn;
   const long long slots = 256LL * (head_dim <= 64 ? 6 : 3);
@@ -95,7 +98,8 @@ void plan_slices(int batch, int q_heads, int kv_heads, int head_dim, int cap, in
     const unsigned sl = ((ucap + n - 1) / n + unit - 1) / unit * unit;
     if (n > 1 && sl < 64) return false;
     const int slices = (int)((ucap + sl - 1) / sl);
-    const double cost = (double)((segs * slices + slots - 1) / slots) * (double)(sl + 100) +
+    const double cost = ((double)((segs * slices + slots - 1) / slots) + (lens ? 0.25 : 0)) *
+                            (double)(sl + 100) +
                         (slices > 1 ? 75 : 0) +
                         (slices > 32 ? (paged ? 3.5 : 4.5) * slices : 0);
     if (!*nsplit || cost < best) {
@@ -144,11 +148,31 @@ extern "C" size_t tm_decode_attention_full_workspace_size(int batch, int q_heads
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || head_dim <= 0 ||
       seq_len <= 0)
     return 0;
+  int most = 1;
+  for (const bool lens : {false, true}) {
+    int ns = 1, sl = 0;
+    plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, page_size > 0 ? page_size : 1,
+                page_size > 0, lens, &ns, &sl);
+    most = std::max(most, ns);
+  }
+  return std::max(base, most > 1 ? (size_t)batch * q_heads * most * (head_dim + 4) * sizeof(float)
+                                 : (size_t)0);
+}
+
+extern "C" int tm_decode_attention_plan(int batch, int q_heads, int kv_heads, int head_dim,
+                                        int seq_len, int page_size, int own_lengths, int* slices,
+                                        int* slice_positions) {
+  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || head_dim <= 0 ||
+      seq_len <= 0)
+    return fail(TM_ERR_INVALID_ARG, "tm_decode_attention_plan: batch=%d q_heads=%d kv_heads=%d "
+                "head_dim=%d seq_len=%d", batch, q_heads, kv_heads, head_dim, seq_len);
+  clear_error();
   int ns = 1, sl = 0;
   plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, page_size > 0 ? page_size : 1,
-              page_size > 0, &ns, &sl);
-  return std::max(base, ns > 1 ? (size_t)batch * q_heads * ns * (head_dim + 4) * sizeof(float)
-                               : (size_t)0);
+              page_size > 0, own_lengths != 0, &ns, &sl);
+  if (slices) *slices = ns;
+  if (slice_positions) *slice_positions = sl;
+  return 0;
 }
 
 // Both entry points.  noalloc: the slice partials go to the device's
@@ -220,7 +244,8 @@ static int decode_attention(const char* op, bool noalloc, const void* q, const v
     const size_t per = (size_t)batch * q_heads * (head_dim + 4) * sizeof(float);
     bool full = !f32 && !noalloc && workspace && aligned16(workspace);
     if (full) {
-      plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged, &ns, &sl);
+      plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged,
+                  seq_lens != nullptr, &ns, &sl);
       full = ns == 1 || workspace_bytes >= per * ns;
     }
     if (!full) plan_split(batch, q_heads, kv_heads, seq_len, p.page_size, paged, &ns, &sl);
@@ -240,14 +265,17 @@ static int decode_attention(const char* op, bool noalloc, const void* q, const v
       workspace_bytes = bytes;
     }
     if (ns > 1 && (!workspace || workspace_bytes < need || !aligned16(workspace))) {
-      // no room for slice partials: one slice per wave (paged: only while it
-      // spans at most 64 pages)
+      // no room for slice partials: one slice per wave (paged: only while it spans at
+      // most 64 pages, the fp32 kernel's limit.  The 16-bit kernel walks any number, 7
+      // to 14 times as fast as the general one, but rounds the probabilities to 16
+      // bits, which these calls have always had in fp32.)
       ns = 1;
       sl = (seq_len + 31) / 32 * 32;
       if (paged && (long long)sl > 64LL * page_size) mfma = false;
     }
     if (mfma) {
       p.nsplit = ns; p.split_len = sl;
+      p.slice_unit = slice_unit(page_size, paged);
       p.ws = (float*)workspace;
       const int group = q_heads / kv_heads, hbn = (group + 15) / 16;
       // [head dim][cache dtype][query dtype other than the cache's: hi + lo split]

@@ -51,6 +51,7 @@ struct DecodeParams {
   int page_shift;           // log2(page_size) when a power of two, else -1
   int nsplit, split_len;    // slices of split_len positions (paged: whole
                             // pages; fp32 caches at most 64 of them)
+  int slice_unit;           // what slices are a multiple of: 32 and whole pages
   float sl2;                // scale * log2(e)
   int q_dt, kv_dt, o_dt;    // TM_DT_* codes
 };
@@ -100,6 +101,18 @@ TM_DEV int seq_len_of(const DecodeParams& p, int b) {
   return p.seq_lens ? min(p.seq_lens[b], p.seq_len) : p.seq_len;
 }
 
+// Positions of each slice of a sequence: with lengths of their own, its own length in
+// nsplit equal parts.  A wave streams its slice at a latency-bound rate (about 60 ns a
+// position), so slices of the capacity's split_len would leave a short sequence to one
+// wave.  us, slices of split_len -> here, all sequences a quarter full: 16 of 8192 (6
+// slices) 97 -> 37, 23 of 8727 (4) 121 -> 45; from a quarter to all full 108 -> 106, 137 ->
+// 132; all full 112 and 141 in both.
+TM_DEV int slice_len(const DecodeParams& p, int len) {
+  if (!p.seq_lens || p.nsplit == 1) return p.split_len;
+  const int n = p.nsplit, u = p.slice_unit;
+  return min(p.split_len, ((max(len, 0) + n - 1) / n + u - 1) / u * u);
+}
+
 TM_DEV float ld_any(const void* ptr, long long i, int dt) {
   if (dt == TM_DT_F32) return ((const float*)ptr)[i];
   if (dt == TM_DT_F16) return f16_bits_to_f32(((const uint16_t*)ptr)[i]);
@@ -146,7 +159,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeParams& p) {
   const int split = blockIdx.x, b = blockIdx.z;
   const int kvh = blockIdx.y / hbn, hb = blockIdx.y - kvh * hbn;
   const int len = seq_len_of(p, b);
-  const int p0 = split * p.split_len, p1 = min(len, p0 + p.split_len);
+  const int sl = slice_len(p, len), p0 = split * sl, p1 = min(len, p0 + sl);
   const int hq = kvh * group + 16 * hb + l16;    // this lane's query head
   const bool hvalid = 16 * hb + l16 < group;
 

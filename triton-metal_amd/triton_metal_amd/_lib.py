@@ -69,6 +69,8 @@ SIGNATURES = {
     "tm_kda_compact_workspace_size": [i32, i32, i32, i32, i32, i32],
     "tm_decode_attention_workspace_size": [i32, i32, i32, i32, i32, i32],
     "tm_decode_attention_full_workspace_size": [i32, i32, i32, i32, i32, i32],
+    "tm_decode_attention_plan": [i32, i32, i32, i32, i32, i32, i32, C.POINTER(i32),
+                                 C.POINTER(i32)],
     "tm_decode_attention": [vp, vp, vp, vp, vp, i32, i32, i32, i32, vp, i32,
                             C.POINTER(C.c_longlong), vp, i32, i32, C.c_float, i32, i32, i32, vp,
                             sz, vp],
