@@ -47,7 +47,8 @@ def _sum_bound(x, deq, mag):
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ACT)
 @pytest.mark.parametrize("qbits,zeros", [(4, None), (4, "s"), (4, "u"), (8, None)])
-@pytest.mark.parametrize("M,N,K", [(1, 144, 640), (2, 48, 128), (40, 272, 1152), (64, 128, 384),
+@pytest.mark.parametrize("M,N,K", [(1, 144, 640), (2, 48, 128), (1, 4112, 640), (2, 4112, 128),
+                                   (9, 144, 384), (40, 272, 1152), (64, 128, 384),
                                    (65, 400, 896), (129, 16, 2176), (200, 1040, 3200),
                                    (1300, 2064, 384)])
 def test_against_the_fp32_product(qbits, zeros, act, M, N, K):
@@ -56,7 +57,8 @@ def test_against_the_fp32_product(qbits, zeros, act, M, N, K):
     if not (qbits == 4 and M == 1):
         name = tm.wq_kernel_for(qbits, M, N, K, act_dtype=dt, details=True, zero_dtype=None if z is
                                 None else z.dtype)["name"]
-        assert name == f"wq_pipe_q{qbits}_{act}_z{zeros or 'n'}_r{1 if M <= 64 else 2}", name
+        assert name == (f"wq_pipe_q{qbits}_{act}_z{zeros or 'n'}_r{1 if M <= 64 else 2}"
+                        if M > 2 or N > 4096 else "wq_general"), name
     bias = torch.randn(N).to(dt)
     xd, wd, sd, bd = x.cuda(), w.cuda(), s.cuda(), bias.cuda()
     zd = None if z is None else z.cuda()
@@ -219,6 +221,11 @@ def test_selection():
     assert k(4, 1000, 4096, 11008, zero_dtype=u8)["name"] == "wq_pipe_q4_f16_zu_r2"
     assert k(4, 1000, 4096, 4096, zero_dtype=u8)["name"].startswith("wq_wide_")
     assert k(8, 40, 1280, 3456)["name"] == "wq_pipe_q8_f16_zn_r1"
+    # few rows and columns, on both sides
+    pipe = lambda *a, **kw: k(*a, **kw)["name"].startswith("wq_pipe_")
+    assert pipe(8, 1, 4112, 640) and not pipe(8, 1, 4096, 640) and not pipe(8, 1, 4096, 2432)
+    assert pipe(4, 9, 2448, 384) and not pipe(4, 8, 2448, 384) and not pipe(8, 8, 272, 384)
+    assert pipe(4, 5, 272, 128) and not pipe(4, 4, 272, 128) and pipe(8, 3, 272, 128)
     # without the workspace int4 stays where it was
     assert k(4, 228, 2816, 7040, with_workspace=False)["name"] == "wq_general"
     assert k(8, 700, 22016, 4096, with_workspace=False)["workspace_bytes"] == 0

@@ -337,8 +337,16 @@ void wq_plan(int qbits, int M, int N, int K, int G, int adt, int sdt, int zdt, u
   // that is a multiple of 256 only: larger weights (M = 3 K = 3840 N = 11520 28
   // -> 19; M = 228 K = 2816 N = 2816 26 -> 23, smaller ones lose
   // what the permuting launch and the reduction cost, 4)
-  if (pipe_ok && (K % 256 != 0 || N % 64 != 0 ||
-                  (K <= 4096 && M > 1 && (long long)N * K >= (M > 64 ? 5000000 : 20000000))) &&
+  // wq_general keeps a few rows of up to 4096 columns, where its one wave per column
+  // ends before a tile's serial k steps do (us, general / pipelined): int8 M = 1 N = 272 K = 640
+  // 4.8 / 9.1, N = 2448 K = 1152 6.8 / 11.4, K = 2432 9.8 / 12.0, N = 8192 K = 640 9.5 / 7.9;
+  // int4 N = 2448 K = 384 M = 2 5.0 / 7.4, M = 8 6.6 / 8.1, M = 16 10.2 / 8.1, K = 128 M = 4
+  // 5.5 / 6.4, M = 8 6.6 / 6.5; int8 N = 272 K = 384 M = 8 5.7 / 5.8, K = 128 M = 4 4.9 / 4.7
+  const bool general = (K % 256 != 0 || N % 64 != 0) && N <= 4096 &&
+                       (M == 1 || (K <= 384 && M <= (K > 256 ? 8 : qbits == 4 ? 4 : 2)));
+  if (pipe_ok && !general &&
+      (K % 256 != 0 || N % 64 != 0 ||
+       (K <= 4096 && M > 1 && (long long)N * K >= (M > 64 ? 5000000 : 20000000))) &&
       pipe())
     return;
   // tiled kernel: 64 x 64 output tiles walking K in steps of 256.  With a
