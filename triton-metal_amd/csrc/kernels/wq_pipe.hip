@@ -285,6 +285,8 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
   const uint32_t eb = lds0 + (uint32_t)wave * 32 * LDW * 4;
   const int mw = m0 + 32 * RT * wm, nw = n0 + 32 * CT * wn;
   float* P = p.P ? p.P + (size_t)blockIdx.y * p.M * p.N : nullptr;
+  constexpr int LPR = 4 * CT, NP = 2 * CT;  // lanes of a row, pieces of 8 columns per lane
+  f4_t size = {0.f, 0.f, 0.f, 0.f};         // infinite or NaN: so is one of the outputs
   static_for<0, RT>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
 #pragma unroll
@@ -296,7 +298,6 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
         else v = sc[j] * acc[i][j][e];
         *(lds_f_t*)(eb + 4u * ((8 * (e >> 2) + 4 * h + (e & 3)) * LDW + 32 * j + l32)) = v;
       }
-    constexpr int LPR = 4 * CT, NP = 2 * CT;
     const int c = 8 * (lane % LPR), n = nw + c;  // N % 16 == 0: whole pieces
 #pragma unroll
     for (int t = 0; t < NP; ++t) {
@@ -305,25 +306,8 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
       f4_t b = *(lds_f4_t*)(eb + 4u * (r * LDW + c + 4));
       const bool in = m < p.M && n < p.N;
       if constexpr (!LESS) {
-        // infinite and NaN outputs again as wq_general sums them (wq_direct)
-        bool bad = false;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) bad |= not_finite(a[e]) || not_finite(b[e]);
-        for (uint64_t todo = __ballot(in && bad); todo; todo &= todo - 1) {
-          const int l = __builtin_ctzll(todo), ml = __builtin_amdgcn_readlane(m, l),
-                    nl = __builtin_amdgcn_readlane(n, l);
-          for (int e = 0; e < 8; ++e) {
-            const float v = e < 4 ? a[e & 3] : b[e & 3];
-            if (!((__ballot(not_finite(v)) >> l) & 1)) continue;
-            const float d = wq_direct<QB, BF16, ZDT>(
-                p.X0 + (size_t)ml * K, p.W + (size_t)(nl + e) * wrow, p.S, p.Z,
-                (size_t)(nl + e) * (QB == 4 ? ng : 1), k0, k1, lane);
-            if (lane == l) {
-              if (e < 4) a[e & 3] = d;
-              else b[e & 3] = d;
-            }
-          }
-        }
+        for (int e = 0; e < 4; ++e) size[e] += __builtin_fabsf(a[e]) + __builtin_fabsf(b[e]);
       }
       if (!in) continue;
       const size_t o = (size_t)m * p.N + n;
@@ -336,6 +320,33 @@ __device__ __forceinline__ void wq_pipe_body(const WqPipeParams& p) {
       }
     }
   });
+  if constexpr (!LESS) {
+    // outputs that came out infinite or NaN again, as wq_general sums them
+    // (wq_direct), piece by piece by the whole wave; the lane that holds the piece
+    // reads back what it stored.  One sum of sizes finds them, and the code stands
+    // in one place: a test of each output cost every call 0.4 us.
+    for (uint64_t todo = __ballot(not_finite((size[0] + size[1]) + (size[2] + size[3]))); todo;
+         todo &= todo - 1) {
+      const int l = __builtin_ctzll(todo), n = nw + 8 * (l % LPR);
+      if (n >= p.N) continue;
+#pragma unroll 1
+      for (int x = 0; x < RT * NP * 8; ++x) {
+        const int e = x & 7, t = x >> 3;
+        const int m = mw + 32 * (t / NP) + (t % NP) * (64 / LPR) + l / LPR;
+        if (m >= p.M) break;  // (rows rise with t)
+        const size_t o = (size_t)m * p.N + n + e;
+        bool bad = false;
+        if (lane == l) bad = not_finite(P ? P[o] : load_as_f32<SDT>(p.Y, o));
+        if (!__ballot(bad)) continue;
+        const float d = wq_direct<QB, BF16, ZDT>(
+            p.X0 + (size_t)m * K, p.W + (size_t)(n + e) * wrow, p.S, p.Z,
+            (size_t)(n + e) * (QB == 4 ? ng : 1), k0, k1, lane);
+        if (lane != l) continue;
+        if (P) P[o] = d;
+        else store_as_f32_rt(p.Y, o, SDT, d + (p.bias ? load_as_f32<SDT>(p.bias, n + e) : 0.0f));
+      }
+    }
+  }
 }
 
 // wq_pipe_q<bits>_<act>_z<zeros>_r<RT>
