@@ -242,15 +242,21 @@ static int decode_attention(const char* op, bool noalloc, const void* q, const v
   if (mfma) {
     int ns = 1, sl = 0;
     const size_t per = (size_t)batch * q_heads * (head_dim + 4) * sizeof(float);
-    bool full = !f32 && !noalloc && workspace && aligned16(workspace);
-    if (full) {
+    // noalloc: as with a workspace of tm_decode_attention_workspace_size bytes
+    plan_split(batch, q_heads, kv_heads, seq_len, p.page_size, paged, &ns, &sl);
+    const size_t base = ns > 1 ? per * ns : 0;
+    const size_t have = noalloc ? base : workspace && aligned16(workspace) ? workspace_bytes : 0;
+    if (!f32 && have > 0) {
+      int fns = 1, fsl = 0;
       plan_slices(batch, q_heads, kv_heads, head_dim, seq_len, p.page_size, paged,
-                  seq_lens != nullptr, &ns, &sl);
-      full = ns == 1 || workspace_bytes >= per * ns;
+                  seq_lens != nullptr, &fns, &fsl);
+      if (fns == 1 || have >= per * fns) {
+        ns = fns;
+        sl = fsl;
+      }
     }
-    if (!full) plan_split(batch, q_heads, kv_heads, seq_len, p.page_size, paged, &ns, &sl);
-    const size_t need = per * ns;
-    if (noalloc && ns > 1) {
+    const size_t need = noalloc ? base : per * ns;
+    if (noalloc && base > 0) {
       static DeviceGlobal scratch("tm_decode_scratch");
       void* ptr = nullptr;
       size_t bytes = 0;
