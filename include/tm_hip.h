@@ -142,11 +142,15 @@ int tm_int4_linear(const void* input, const void* weight, const void* bias, void
  * group_size ignored for int8) with a caller-provided device workspace:
  * shapes whose kernel would leave the GPU underfilled or exceed a kernel's K
  * (long-K down projections at M >= 17, int8 K > 16384, ...) then run split-K
- * (fp32 slice sums in the workspace, then one reduction launch).  workspace:
- * 16-byte aligned, at least tm_wq_workspace_bytes(...) bytes, used only by
+ * (fp32 slice sums in the workspace, then one reduction launch), and int4 products
+ * of many tiles or of a K that is a multiple of 128 only the pipelined kernels, which
+ * keep there a copy of the input in their operands' order and its group sums
+ * (2 M K + M K / 32 bytes and up).  workspace:
+ * 16-byte aligned, at least tm_wq_workspace_bytes(...) bytes (with a smaller
+ * one the pipelined kernels give way to others; a split-K call fails), used only by
  * this call's launches on `stream` (overlapping calls must not share one);
  * NULL / 0 behaves as tm_int4_matmul / tm_int8_matmul / the linear forms, which
- * never split.  The Python operators (int4_matmul, ...) pass a torch-allocated
+ * need none.  The Python operators (int4_matmul, ...) pass a torch-allocated
  * workspace this way.  No counterpart in the reference, whose templates run
  * one threadgroup per output tile over the whole of K. */
 int tm_wq_matmul_ws(int qbits, const void* input, const void* weight, const void* bias,
@@ -154,15 +158,16 @@ int tm_wq_matmul_ws(int qbits, const void* input, const void* weight, const void
                     int group_size, int act_dtype, int scale_dtype, int zero_dtype,
                     void* workspace, size_t workspace_bytes, void* stream);
 /* Workspace bytes tm_wq_matmul_ws needs for this call on the current device
- * (0: no split-K; then any workspace, or none, will do).  The pointers are
+ * (0: any workspace, or none, will do).  The pointers are
  * only inspected for their alignment. */
 size_t tm_wq_workspace_bytes(int qbits, const void* input, const void* weight,
                              const void* scales, const void* zeros, int M, int N, int K,
                              int group_size, int act_dtype, int scale_dtype, int zero_dtype);
 /* Kernel selection of the entry points above, without launching: the name of
  * the gfx950 kernel a call with these sizes and dtypes would run, its grid,
- * block and dynamic LDS bytes, its k-slices (1: no split-K; the grid is then
- * (grid, splits) and wq_splitk_reduce_<act> follows) and workspace bytes,
+ * block and dynamic LDS bytes, its k-slices (more than 1: the grid is
+ * (grid, splits) and wq_splitk_reduce_<act> follows; int4 wq_pipe_* kernels run behind
+ * wq_pipe_prep_<act>) and workspace bytes,
  * for a device with cu_count CUs and max_lds bytes of dynamic LDS per
  * workgroup (MI355X: 256, 163840), with or without a workspace.  align_flags:
  * TM_WQ_ALIGN_* bits for the pointer alignments of the call.  A diagnostic with

@@ -35,7 +35,7 @@ struct MmParams {
 // full MFMA load allow); `res` tiles share a CU; fixed ns per round for the
 // pipeline's fill and the epilogue.  The larger tile moves fewer bytes into LDS
 // per MFMA, the smaller ones leave less of the last round idle and wait less
-// where there are few tiles: us for 44 / 42 / 22 / 22d / 21 / 11, weights and
+// where there are few tiles (256 CUs, the whole chip): us for 44 / 42 / 22 / 22d / 21 / 11, weights and
 // activations coming from HBM
 //   4096 x 4096 x 4096    117 / 137 / 144 / 159 / 179 / 234
 //   2000 x 11008 x 4096   231 / 222 / 241 / 264 / 292 / 360

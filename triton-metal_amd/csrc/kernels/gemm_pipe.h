@@ -21,7 +21,8 @@
 // the power limit), copies alone 0.88, all of it 1.49; the rest is 13 us per round
 // of tiles (first copies, C).  us, kernels it replaced -> this: fp16 2000 x 11008
 // x 4096 260 -> 196, e4m3 2048 x 4096 x 4096 178 -> 59, transposed A with add-
-// matrix 4096 x 4096 x 2000 204 -> 86, 4096^3 113 -> 107.
+// matrix 4096 x 4096 x 2000 204 -> 86.  (Aligned products whose 256-tiles fill the
+// chip keep gemm_t256: 4096^3 on one set of buffers 118, here 123.)
 #pragma once
 #include "common.h"
 

@@ -1,5 +1,5 @@
 // Weight-only matmul on pipelined MFMA tiles, for the sizes the streaming and
-// wide kernels do not take (K a multiple of 128 only, any M and N) and for
+// wide kernels do not take (K a multiple of 128 only, any M and N % 16 == 0) and for
 // products large enough to fill the chip with 128 x 128 tiles:
 //
 //   Y[m, n] = sum_k X[m, k] (q(n, k) - z(n, g)) s(n, g)   (+ bias[n])
